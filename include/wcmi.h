@@ -408,6 +408,22 @@ typedef struct wc_path_rows {
 int wc_paths_emit(const wc_scene* scene, const wc_solve* solve, const int* row_offset, const int* path_count,
                   const wc_path_rows* rows, void* stream);
 
+/* The same count and rows from the radiomap's visibility masks (chain validity
+ * and edge visibility kernels over `tiles`, as wc_radiomap_forward takes
+ * them), instead of testing every candidate of a cell in one lane, twice.
+ * `workspace` (wc_paths_masks_workspace_bytes) carries the masks from the
+ * count to the emit. path_count also counts visible edges whose field falls
+ * below the gain floor; the emit writes such a row with path_length_m NaN,
+ * which the canonical compaction drops. row_list: scratch of total + 2 ints,
+ * total = the sum of path_count. Rows kept by the compaction are those of
+ * wc_paths_count / wc_paths_emit, in the same order. */
+size_t wc_paths_masks_workspace_bytes(int cells, int lanes_per_cell, int edge_count, int max_tx_chains, int tx_count);
+int wc_paths_count_masked(const wc_scene* scene, const wc_solve* solve, void* workspace, const int* tiles,
+                          int tile_count, int* path_count, void* stream);
+int wc_paths_emit_masked(const wc_scene* scene, const wc_solve* solve, void* workspace, const int* tiles,
+                         int tile_count, const int* row_offset, const int* path_count, int total, int* row_list,
+                         const wc_path_rows* rows, void* stream);
+
 int wc_paths_canonical_order(const wc_path_rows* rows, const int* pair_offset, int pair_count, int* permutation,
                              unsigned char* keep, void* stream);
 

@@ -56,6 +56,48 @@ __device__ __forceinline__ int next_set_chain(const ChainMaskView& m, int base, 
     return c1;
 }
 
+// Path record of reflection chain c (depth D) for one receiver; false when
+// the chain does not exist. kLegs: trace the legs (not needed when the chain
+// masks already say they are clear); kRows: fill the interaction sequence.
+template <int D, bool kLegs, bool kRows>
+__device__ __forceinline__ bool reflect_record(const SceneView& s, const wc_solve& q, int c, const V3<float>& tx,
+                                               const V3<float>& rx, const V3<float>& tx_pol, const V3<float>& rx_pol,
+                                               float sqrt_power, float freq, double k_d, PathRecord& rec) {
+    const int* groups = q.chain_groups + c * kMaxDepth;
+    const double* images = q.chain_images + c * kMaxDepth * 3;
+    V3<double> hd[D];
+    int faces[D];
+    if (!solve_chain<D, kLegs>(s, groups, images, tx, rx, hd, faces)) return false;
+    rec.component = kCidRefl;
+    rec.depth = D;
+    rec.candidate = c;
+    rec.edge = -1;
+    V3<float> hf[D], nf[D];
+    int mats[D];
+#pragma unroll
+    for (int b = 0; b < D; ++b) {
+        hf[b] = to_f(hd[b]);
+        double off;
+        nf[b] = to_f(group_normal(s, groups[b], off));
+        mats[b] = s.face_material[faces[b]];
+        if constexpr (kRows) {
+            rec.prim[b] = faces[b];
+            rec.mat[b] = mats[b];
+            rec.pos[b][0] = hf[b].x; rec.pos[b][1] = hf[b].y; rec.pos[b][2] = hf[b].z;
+            rec.nrm[b][0] = nf[b].x; rec.nrm[b][1] = nf[b].y; rec.nrm[b][2] = nf[b].z;
+        }
+    }
+    const V3<double> img{images[3 * (D - 1)], images[3 * (D - 1) + 1], images[3 * (D - 1) + 2]};
+    rec.length_d = norm(to_d(rx) - img);
+    rec.length = (float)rec.length_d;
+    V3<float> arrival, departure;
+    const C3<float> v = reflection_field<D>(s, tx, rx, hf, nf, mats, tx_pol, freq, k_d, rec.length_d, arrival,
+                                            departure);
+    finish_record(rec, v, arrival, rx_pol, sqrt_power);
+    rec.dep[0] = departure.x; rec.dep[1] = departure.y; rec.dep[2] = departure.z;
+    return true;
+}
+
 // Reflection chains of one compile-time depth D for one cell. With a chain
 // mask (from chain_visibility_kernel) only the chains whose legs are all
 // clear are visited and their legs are not traced again.
@@ -70,39 +112,9 @@ __device__ __forceinline__ void reflect_depth(const SceneView& s, const wc_solve
     for (int c = kMasked ? next_set_chain(chain_mask, base, c0, c1) : c0 + sub; c < c1;
          c = kMasked ? next_set_chain(chain_mask, base, c + 1, c1) : c + stride) {
         if (kMasked && (c - c0) % stride != sub) continue;
-        const int* groups = q.chain_groups + c * kMaxDepth;
-        const double* images = q.chain_images + c * kMaxDepth * 3;
-        V3<double> hd[D];
-        int faces[D];
-        if (!solve_chain<D, !kMasked>(s, groups, images, tx, rx, hd, faces)) continue;
         PathRecord rec;
-        rec.component = kCidRefl;
-        rec.depth = D;
-        rec.candidate = c;
-        rec.edge = -1;
-        V3<float> hf[D], nf[D];
-        int mats[D];
-#pragma unroll
-        for (int b = 0; b < D; ++b) {
-            hf[b] = to_f(hd[b]);
-            double off;
-            nf[b] = to_f(group_normal(s, groups[b], off));
-            mats[b] = s.face_material[faces[b]];
-            if constexpr (Sink::kNeedsRows) {
-                rec.prim[b] = faces[b];
-                rec.mat[b] = mats[b];
-                rec.pos[b][0] = hf[b].x; rec.pos[b][1] = hf[b].y; rec.pos[b][2] = hf[b].z;
-                rec.nrm[b][0] = nf[b].x; rec.nrm[b][1] = nf[b].y; rec.nrm[b][2] = nf[b].z;
-            }
-        }
-        const V3<double> img{images[3 * (D - 1)], images[3 * (D - 1) + 1], images[3 * (D - 1) + 2]};
-        rec.length_d = norm(to_d(rx) - img);
-        rec.length = (float)rec.length_d;
-        V3<float> arrival, departure;
-        const C3<float> v = reflection_field<D>(s, tx, rx, hf, nf, mats, tx_pol, freq, k_d, rec.length_d, arrival,
-                                                departure);
-        finish_record(rec, v, arrival, rx_pol, sqrt_power);
-        rec.dep[0] = departure.x; rec.dep[1] = departure.y; rec.dep[2] = departure.z;
+        if (!reflect_record<D, !kMasked, Sink::kNeedsRows>(s, q, c, tx, rx, tx_pol, rx_pol, sqrt_power, freq, k_d, rec))
+            continue;
         sink.path(rec);
     }
 }
@@ -144,6 +156,86 @@ __device__ __forceinline__ bool edge_visible(const SceneView& s, const Edge& e, 
     return true;
 }
 
+__device__ __forceinline__ void los_record(const V3<float>& dir, const V3<float>& tx_pol, const V3<float>& rx_pol,
+                                           float sqrt_power, float k, double k_d, double dist_d, PathRecord& rec) {
+    rec.component = kCidLos;
+    rec.depth = 0;
+    rec.candidate = -1;
+    rec.edge = -1;
+    rec.length_d = dist_d;
+    rec.length = (float)dist_d;
+    const C3<float> v = los_field(dir, tx_pol, k, k_d, dist_d);
+    finish_record(rec, v, dir, rx_pol, sqrt_power);
+    rec.dep[0] = dir.x; rec.dep[1] = dir.y; rec.dep[2] = dir.z;
+}
+
+// Transmission through the d walls `hits` of the straight segment.
+template <bool kRows>
+__device__ __forceinline__ void transmission_record(const SceneView& s, int d, const Hit* hits, const V3<float>& tx,
+                                                    const V3<float>& seg, const V3<float>& dir,
+                                                    const V3<float>& tx_pol, const V3<float>& rx_pol,
+                                                    float sqrt_power, float freq, double k_d, double dist_d,
+                                                    PathRecord& rec) {
+    rec.component = kCidTrans;
+    rec.depth = d;
+    rec.candidate = -1;
+    rec.edge = -1;
+    V3<float> normals[kMaxHits];
+    const C3<float> v = transmission_field(s, d, hits, dir, tx_pol, freq, k_d, dist_d, rec.mat, normals);
+    if constexpr (kRows) {
+        for (int w = 0; w < d; ++w) {
+            rec.prim[w] = hits[w].face;
+            const float tt = hits[w].t;
+            rec.pos[w][0] = tx.x + seg.x * tt; rec.pos[w][1] = tx.y + seg.y * tt;
+            rec.pos[w][2] = tx.z + seg.z * tt;
+            rec.nrm[w][0] = normals[w].x; rec.nrm[w][1] = normals[w].y; rec.nrm[w][2] = normals[w].z;
+        }
+    }
+    rec.length_d = dist_d;
+    rec.length = (float)dist_d;
+    finish_record(rec, v, dir, rx_pol, sqrt_power);
+    rec.dep[0] = dir.x; rec.dep[1] = dir.y; rec.dep[2] = dir.z;
+}
+
+// Diffraction at edge ei with its geometry g; false below the gain floor
+// (the record is complete either way).
+template <bool kRows>
+__device__ __forceinline__ bool diffraction_record(const SceneView& s, const Edge& e, int ei, const DiffGeometry& g,
+                                                   const V3<float>& tx, const V3<float>& rx, const V3<float>& tx_pol,
+                                                   const V3<float>& rx_pol, float sqrt_power, float freq, double k_d,
+                                                   PathRecord& rec) {
+    rec.component = kCidDiff;
+    rec.depth = 1;
+    rec.candidate = ei;
+    rec.edge = ei;
+    if constexpr (kRows) {
+        rec.prim[0] = ei;
+        rec.mat[0] = e.material0;
+        rec.pos[0][0] = (float)g.q.x; rec.pos[0][1] = (float)g.q.y; rec.pos[0][2] = (float)g.q.z;
+        rec.nrm[0][0] = e.n0x; rec.nrm[0][1] = e.n0y; rec.nrm[0][2] = e.n0z;
+    }
+    rec.length_d = g.s + g.sp;
+    rec.length = (float)rec.length_d;
+    V3<float> arrival, departure;
+    const C3<float> v = diffraction_field(s, e, g, tx, rx, tx_pol, freq, k_d, arrival, departure);
+    finish_record(rec, v, arrival, rx_pol, sqrt_power);
+    rec.dep[0] = departure.x; rec.dep[1] = departure.y; rec.dep[2] = departure.z;
+    return rec.gain >= kGainFloor;
+}
+
+// Walls of the straight segment of one (transmitter, receiver) pair: the
+// ordered hits when transmission is requested (count returned; max_depth + 1
+// when there are more), else 1 when anything blocks it and 0 when it is clear.
+__device__ __forceinline__ int straight_hits(const SceneView& s, int comps, int max_depth, const V3<float>& tx,
+                                             const V3<float>& seg, double dist_d, Hit* hits) {
+    const float len = (float)dist_d;
+    if (!(comps & (kCompLos | kCompTrans)) || !(len > 2.0f * kSegmentBias)) return 0;
+    const float eps = kSegmentBias / len;
+    const RayPre r = ray_setup(tx.x, tx.y, tx.z, seg.x, seg.y, seg.z);
+    if (comps & kCompTrans) return gather_hits(s, r, eps, 1.0f - eps, max_depth, hits);
+    return occluded(s, r, eps, 1.0f - eps, -1, -1) ? 1 : 0;
+}
+
 // Passes of the fused evaluation: all components (row export), the
 // non-diffraction components, or diffraction only. Splitting the radiomap
 // into two launches gives each its own register budget.
@@ -178,29 +270,10 @@ __device__ void eval_cell(const SceneView& s, const wc_solve& q, int t, int cell
     const V3<float> seg = rx - tx;
     const double dist_d = norm(to_d(rx) - to_d(tx));
     const V3<float> dir = safe_normalize(seg, v3c<float>(0.f, 0.f, 1.f));
-    if (kMain && sub == 0 && (comps & (kCompLos | kCompTrans))) {
-        const float len = (float)dist_d;
-        if (len > 2.0f * kSegmentBias) {
-            const float eps = kSegmentBias / len;
-            const RayPre r = ray_setup(tx.x, tx.y, tx.z, seg.x, seg.y, seg.z);
-            if (comps & kCompTrans) {
-                nh = gather_hits(s, r, eps, 1.0f - eps, max_depth, hits);
-            } else {
-                nh = occluded(s, r, eps, 1.0f - eps, -1, -1) ? 1 : 0;
-            }
-        }
-    }
+    if (kMain && sub == 0) nh = straight_hits(s, comps, max_depth, tx, seg, dist_d, hits);
     if (kMain && sub == 0 && (comps & kCompLos) && nh == 0) {
         PathRecord rec;
-        rec.component = kCidLos;
-        rec.depth = 0;
-        rec.candidate = -1;
-        rec.edge = -1;
-        rec.length_d = dist_d;
-        rec.length = (float)dist_d;
-        const C3<float> v = los_field(dir, tx_pol, k, k_d, dist_d);
-        finish_record(rec, v, dir, rx_pol, sqrt_power);
-        rec.dep[0] = dir.x; rec.dep[1] = dir.y; rec.dep[2] = dir.z;
+        los_record(dir, tx_pol, rx_pol, sqrt_power, k, k_d, dist_d, rec);
         sink.path(rec);
     }
     if (kMain && sub == 0 && (comps & kCompTrans) && (comps & kStrictPenetration) && nh > max_depth)
@@ -238,47 +311,16 @@ __device__ void eval_cell(const SceneView& s, const wc_solve& q, int t, int cell
                 if (!diffraction_geometry(e, tx, rx, g)) continue;
                 if (!diff_mask && !edge_visible(s, e, g, tx, rx)) continue;
                 PathRecord rec;
-                rec.component = kCidDiff;
-                rec.depth = 1;
-                rec.candidate = ei;
-                rec.edge = ei;
-                if constexpr (Sink::kNeedsRows) {
-                    rec.prim[0] = ei;
-                    rec.mat[0] = e.material0;
-                    rec.pos[0][0] = (float)g.q.x; rec.pos[0][1] = (float)g.q.y; rec.pos[0][2] = (float)g.q.z;
-                    rec.nrm[0][0] = e.n0x; rec.nrm[0][1] = e.n0y; rec.nrm[0][2] = e.n0z;
-                }
-                rec.length_d = g.s + g.sp;
-                rec.length = (float)rec.length_d;
-                V3<float> arrival, departure;
-                const C3<float> v = diffraction_field(s, e, g, tx, rx, tx_pol, freq, k_d, arrival, departure);
-                finish_record(rec, v, arrival, rx_pol, sqrt_power);
-                if (!(rec.gain >= kGainFloor)) continue;
-                rec.dep[0] = departure.x; rec.dep[1] = departure.y; rec.dep[2] = departure.z;
+                if (!diffraction_record<Sink::kNeedsRows>(s, e, ei, g, tx, rx, tx_pol, rx_pol, sqrt_power, freq, k_d,
+                                                          rec))
+                    continue;
                 sink.path(rec);
             }
         }
         if (kMain && sub == 0 && (comps & kCompTrans) && nh == d) {
             PathRecord rec;
-            rec.component = kCidTrans;
-            rec.depth = d;
-            rec.candidate = -1;
-            rec.edge = -1;
-            V3<float> normals[kMaxHits];
-            const C3<float> v = transmission_field(s, d, hits, dir, tx_pol, freq, k_d, dist_d, rec.mat, normals);
-            if constexpr (Sink::kNeedsRows) {
-                for (int w = 0; w < d; ++w) {
-                    rec.prim[w] = hits[w].face;
-                    const float tt = hits[w].t;
-                    rec.pos[w][0] = tx.x + seg.x * tt; rec.pos[w][1] = tx.y + seg.y * tt;
-                    rec.pos[w][2] = tx.z + seg.z * tt;
-                    rec.nrm[w][0] = normals[w].x; rec.nrm[w][1] = normals[w].y; rec.nrm[w][2] = normals[w].z;
-                }
-            }
-            rec.length_d = dist_d;
-            rec.length = (float)dist_d;
-            finish_record(rec, v, dir, rx_pol, sqrt_power);
-            rec.dep[0] = dir.x; rec.dep[1] = dir.y; rec.dep[2] = dir.z;
+            transmission_record<Sink::kNeedsRows>(s, d, hits, tx, seg, dir, tx_pol, rx_pol, sqrt_power, freq, k_d,
+                                                  dist_d, rec);
             sink.path(rec);
         }
     }
@@ -332,6 +374,44 @@ struct CellPartial {
 };
 static_assert(sizeof(CellPartial) == 32, "CellPartial layout");
 
+// Row `row` of the path table.
+__device__ __forceinline__ void write_row(const wc_path_rows& rows, int row, int tx, int rx, const PathRecord& r) {
+    const size_t k = (size_t)row;
+    const int w = rows.width;
+    rows.tx_id[k] = tx;
+    rows.rx_id[k] = rx;
+    rows.depth[k] = r.depth;
+    rows.component_id[k] = r.component;
+    rows.edge_id[k] = r.edge;
+    rows.path_length_m[k] = r.length;
+    rows.delay_s[k] = (float)(r.length_d / kC0);
+    rows.path_gain[k] = r.gain;
+    const bool has_seq = r.component != kCidLos;
+    rows.primitive_id[k] = has_seq ? r.prim[0] : -1;
+    rows.material_id[k] = has_seq ? r.mat[0] : -1;
+    for (int j = 0; j < w; ++j) {
+        const bool on = has_seq && j < r.depth;
+        rows.primitive_sequence[k * w + j] = on ? r.prim[j] : -1;
+        rows.material_sequence[k * w + j] = on ? r.mat[j] : -1;
+        for (int c = 0; c < 3; ++c) {
+            rows.interaction_positions[(k * w + j) * 3 + c] = on ? r.pos[j][c] : 0.0f;
+            rows.interaction_normals[(k * w + j) * 3 + c] = on ? r.nrm[j][c] : 0.0f;
+        }
+    }
+    rows.path_field[2 * k] = r.path_field.re;
+    rows.path_field[2 * k + 1] = r.path_field.im;
+    rows.coefficient[2 * k] = r.coefficient.re;
+    rows.coefficient[2 * k + 1] = r.coefficient.im;
+    float* fx = rows.field_xyz + 6 * k;
+    fx[0] = r.field.x.re; fx[1] = r.field.x.im;
+    fx[2] = r.field.y.re; fx[3] = r.field.y.im;
+    fx[4] = r.field.z.re; fx[5] = r.field.z.im;
+    for (int c = 0; c < 3; ++c) {
+        rows.arrival_direction[3 * k + c] = r.arr[c];
+        rows.departure_direction[3 * k + c] = r.dep[c];
+    }
+}
+
 struct EmitSink {
     __device__ void overflow() {}
     static constexpr bool kNeedsRows = true;
@@ -340,41 +420,7 @@ struct EmitSink {
     int row_end;  // rows reserved for this cell by the count pass; never written past
     int tx, rx;
     __device__ void path(const PathRecord& r) {
-        if (row >= row_end) return;
-        const int k = row++;
-        const int w = rows->width;
-        rows->tx_id[k] = tx;
-        rows->rx_id[k] = rx;
-        rows->depth[k] = r.depth;
-        rows->component_id[k] = r.component;
-        rows->edge_id[k] = r.edge;
-        rows->path_length_m[k] = r.length;
-        rows->delay_s[k] = (float)(r.length_d / kC0);
-        rows->path_gain[k] = r.gain;
-        const bool has_seq = r.component != kCidLos;
-        rows->primitive_id[k] = has_seq ? r.prim[0] : -1;
-        rows->material_id[k] = has_seq ? r.mat[0] : -1;
-        for (int j = 0; j < w; ++j) {
-            const bool on = has_seq && j < r.depth;
-            rows->primitive_sequence[k * w + j] = on ? r.prim[j] : -1;
-            rows->material_sequence[k * w + j] = on ? r.mat[j] : -1;
-            for (int c = 0; c < 3; ++c) {
-                rows->interaction_positions[(k * w + j) * 3 + c] = on ? r.pos[j][c] : 0.0f;
-                rows->interaction_normals[(k * w + j) * 3 + c] = on ? r.nrm[j][c] : 0.0f;
-            }
-        }
-        rows->path_field[2 * k] = r.path_field.re;
-        rows->path_field[2 * k + 1] = r.path_field.im;
-        rows->coefficient[2 * k] = r.coefficient.re;
-        rows->coefficient[2 * k + 1] = r.coefficient.im;
-        float* fx = rows->field_xyz + 6 * k;
-        fx[0] = r.field.x.re; fx[1] = r.field.x.im;
-        fx[2] = r.field.y.re; fx[3] = r.field.y.im;
-        fx[4] = r.field.z.re; fx[5] = r.field.z.im;
-        for (int c = 0; c < 3; ++c) {
-            rows->arrival_direction[3 * k + c] = r.arr[c];
-            rows->departure_direction[3 * k + c] = r.dep[c];
-        }
+        if (row < row_end) write_row(*rows, row++, tx, rx, r);
     }
 };
 
@@ -1848,6 +1894,247 @@ __global__ void __launch_bounds__(256) emit_kernel(SceneView s, wc_solve q, cons
     }
 }
 
+// ---- path export from the visibility masks ----------------------------------
+// The rows of a cell are its straight segment (line of sight or the walls it
+// crosses), its valid chains and its visible edges. The radiomap's visibility
+// kernels already answer the last two with many wavefronts per SIMD, so the
+// export runs them once and works on their masks:
+//   1. export_count_kernel: one lane per cell traces the straight segment
+//      (code kept in the workspace) and counts mask bits;
+//   2. export_deal_kernel: one lane per cell walks its bits in canonical order
+//      and leaves (transmitter, receiver, component, candidate) in each row, and
+//      deals the row ids into two lists, diffraction rows from the front and the
+//      others from the back (their order within a list only decides which lane
+//      evaluates a row);
+//   3. export_diff_kernel / export_main_kernel: one lane per row evaluates and
+//      writes it, so a wavefront's 64 rows are neighbouring cells' and every lane
+//      has one path, however unevenly the cells hold them.
+// A visible edge below the gain floor is known only after its field is: its row
+// is written with length NaN, which the canonical compaction never keeps.
+// The per-cell kernels (count_kernel, emit_kernel) test and evaluate every
+// candidate in one lane per cell, twice; on 64 street transmitters with 16 to
+// 4,096 receivers each (0.8 M rows) they took 28.2 + 32.4 ms, and the whole
+// batched solve goes from 57.3 to 3.3 ms with the masks; 32 x 32 endpoints with
+// single reflections (1,024 cells: 16 wavefronts of the per-cell kernels) from
+// 7.3 to 1.6 ms.
+__device__ __forceinline__ int* export_straight(void* workspace) { return static_cast<int*>(workspace); }
+
+// The cell of this lane in tile `tile` (one wavefront per tile; with L lanes
+// per cell a tile holds 64 / L cells, the other lanes idle).
+__device__ __forceinline__ bool export_cell(const wc_solve& q, const int* tiles, int tile, int lane, int& t, int& pos,
+                                            int& cell) {
+    t = tiles[2 * tile];
+    pos = tiles[2 * tile + 1] + lane;
+    if (lane >= 64 / q.lanes_per_cell || pos >= q.cell_offset[t + 1]) return false;
+    cell = cell_at(q, pos);
+    return true;
+}
+
+__device__ __forceinline__ ChainMaskView export_chains(const SceneView& s, const wc_solve& q, void* workspace,
+                                                       int tile, int pos) {
+    ChainMaskView m{nullptr, 0, nullptr};
+    if (q.max_tx_chains > 0) {
+        m.words = chain_masks(workspace, q, s.edge_count) + pos;
+        m.stride = (size_t)q.total_cells;
+        m.touched = touched_bitmaps(workspace, q, s.edge_count) + (size_t)tile * touched_words(q.max_tx_chains);
+    }
+    return m;
+}
+
+__global__ void __launch_bounds__(256) export_count_kernel(SceneView s, wc_solve q, const int* __restrict__ tiles,
+                                                           int tile_count, void* workspace, const unsigned* diff_mask,
+                                                           int* __restrict__ count) {
+    const int lane = threadIdx.x & 63;
+    const int tile = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    if (tile >= tile_count) return;
+    int t, pos, cell;
+    if (!export_cell(q, tiles, tile, lane, t, pos, cell)) return;
+    const V3<float> tx = ld3(q.tx_pos + 3 * t);
+    const V3<float> rx = ld3(q.rx_pos + 3 * (q.rx_shared ? cell - q.cell_offset[t] : cell));
+    const double dist_d = norm(to_d(rx) - to_d(tx));
+    Hit hits[kMaxHits];
+    const int nh = straight_hits(s, q.components, q.max_depth, tx, rx - tx, dist_d, hits);
+    const bool on = nh == 0 ? (q.components & kCompLos) != 0
+                            : (q.components & kCompTrans) != 0 && nh <= q.max_depth;
+    export_straight(workspace)[cell] = on ? nh : -1;
+    int n = on ? 1 : 0;
+    if ((q.components & kCompRefl) && q.max_tx_chains > 0 && q.max_depth > 0) {
+        const ChainMaskView m = export_chains(s, q, workspace, tile, pos);
+        const int words = mask_words(q.max_tx_chains);
+        for (int b = 0; b * 32 < words; ++b)
+            for (unsigned tw = m.touched[b]; tw; tw &= tw - 1)
+                n += __popc(m.words[(size_t)(b * 32 + __ffs(tw) - 1) * m.stride]);
+    }
+    if (diff_mask) {
+        const int words = mask_words(s.edge_count);
+        for (int w = 0; w < words; ++w) n += __popc(diff_mask[(size_t)cell * words + w]);
+    }
+    count[cell] = n;
+}
+
+__global__ void __launch_bounds__(256) export_deal_kernel(SceneView s, wc_solve q, const int* __restrict__ tiles,
+                                                          int tile_count, void* workspace, const unsigned* diff_mask,
+                                                          const int* __restrict__ row_offset,
+                                                          const int* __restrict__ count, wc_path_rows rows, int total,
+                                                          int* __restrict__ list, int* __restrict__ dealt) {
+    const int lane = threadIdx.x & 63;
+    const int tile = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    if (tile >= tile_count) return;
+    int t, pos, cell = 0;
+    const bool live = export_cell(q, tiles, tile, lane, t, pos, cell);
+    const int words = diff_mask ? mask_words(s.edge_count) : 0;
+    int n_diff = 0;
+    if (live)
+        for (int w = 0; w < words; ++w) n_diff += __popc(diff_mask[(size_t)cell * words + w]);
+    const int n_main = live ? count[cell] - n_diff : 0;
+    // the wavefront's shares of the two lists
+    int incl_d = n_diff, incl_m = n_main;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int d = __shfl_up(incl_d, off), m = __shfl_up(incl_m, off);
+        if (lane >= off) {
+            incl_d += d;
+            incl_m += m;
+        }
+    }
+    int base_d = 0, base_m = 0;
+    if (lane == 63) {
+        base_d = atomicAdd(dealt, incl_d);
+        base_m = atomicAdd(dealt + 1, incl_m);
+    }
+    base_d = __shfl(base_d, 63) + incl_d - n_diff;
+    base_m = __shfl(base_m, 63) + incl_m - n_main;
+    if (!live) return;
+    int row = row_offset[cell];
+    const int row_end = row + count[cell];
+    const int rx = cell - q.cell_offset[t];
+    auto deal = [&](int component, int candidate) {
+        if (row >= row_end || row >= total) return;
+        rows.tx_id[row] = t;
+        rows.rx_id[row] = rx;
+        rows.component_id[row] = component;
+        rows.primitive_id[row] = candidate;
+        const int slot = component == kCidDiff ? base_d++ : total - 1 - base_m++;
+        if (slot >= 0 && slot < total) list[slot] = row;
+        ++row;
+    };
+    const int straight = export_straight(workspace)[cell];
+    if (straight == 0) deal(kCidLos, 0);
+    const bool refl = (q.components & kCompRefl) && q.max_tx_chains > 0;
+    const ChainMaskView m = export_chains(s, q, workspace, tile, pos);
+    for (int d = 1; d <= q.max_depth; ++d) {
+        if (refl) {
+            const int base = q.chain_offset[t * kMaxDepth];
+            const int c1 = q.chain_offset[t * kMaxDepth + d];
+            for (int c = next_set_chain(m, base, q.chain_offset[t * kMaxDepth + d - 1], c1); c < c1;
+                 c = next_set_chain(m, base, c + 1, c1))
+                deal(kCidRefl, c);
+        }
+        if (d == 1)
+            for (int w = 0; w < words; ++w)
+                for (unsigned bits = diff_mask[(size_t)cell * words + w]; bits; bits &= bits - 1)
+                    deal(kCidDiff, w * 32 + __ffs(bits) - 1);
+        if (straight == d) deal(kCidTrans, d);
+    }
+}
+
+// Endpoints of a dealt row.
+struct RowEnds {
+    int t, rx_id;
+    V3<float> tx, tx_pol, rx, rx_pol;
+    float sqrt_power;
+};
+__device__ __forceinline__ RowEnds row_ends(const wc_solve& q, const wc_path_rows& rows, int row) {
+    RowEnds e;
+    e.t = rows.tx_id[row];
+    e.rx_id = rows.rx_id[row];
+    e.tx = ld3(q.tx_pos + 3 * e.t);
+    e.tx_pol = ld3(q.tx_pol + 3 * e.t);
+    e.sqrt_power = sqrtf(fmaxf(q.tx_power[e.t], 0.0f));
+    const int rx_index = q.rx_shared ? e.rx_id : q.cell_offset[e.t] + e.rx_id;
+    e.rx = ld3(q.rx_pos + 3 * rx_index);
+    e.rx_pol = ld3(q.rx_pol + 3 * (q.rx_pol_stride ? rx_index : 0));
+    return e;
+}
+
+__global__ void __launch_bounds__(256) export_diff_kernel(SceneView s, wc_solve q, wc_path_rows rows,
+                                                          const int* __restrict__ list,
+                                                          const int* __restrict__ dealt) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= dealt[0]) return;
+    const int row = list[i];
+    const RowEnds ends = row_ends(q, rows, row);
+    const int ei = rows.primitive_id[row];
+    const Edge e = s.edges[ei];
+    PathRecord rec{};
+    DiffGeometry g;
+    const double k_d = q.frequency_hz * kTwoPi / kC0;
+    bool ok = diffraction_geometry(e, ends.tx, ends.rx, g);
+    if (ok) {
+        ok = diffraction_record<true>(s, e, ei, g, ends.tx, ends.rx, ends.tx_pol, ends.rx_pol, ends.sqrt_power,
+                                      (float)q.frequency_hz, k_d, rec);
+    } else {
+        rec.component = kCidDiff;
+        rec.depth = 1;
+        rec.edge = rec.prim[0] = ei;
+    }
+    if (!ok) rec.length = NAN;
+    write_row(rows, row, ends.t, ends.rx_id, rec);
+}
+
+template <int D>
+__device__ __forceinline__ bool export_chain(const SceneView& s, const wc_solve& q, const RowEnds& ends, int c,
+                                             float freq, double k_d, PathRecord& rec) {
+    return reflect_record<D, false, true>(s, q, c, ends.tx, ends.rx, ends.tx_pol, ends.rx_pol, ends.sqrt_power, freq,
+                                          k_d, rec);
+}
+
+__global__ void __launch_bounds__(256) export_main_kernel(SceneView s, wc_solve q, wc_path_rows rows, int total,
+                                                          const int* __restrict__ list,
+                                                          const int* __restrict__ dealt) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= dealt[1]) return;
+    const int row = list[total - 1 - i];
+    const RowEnds ends = row_ends(q, rows, row);
+    const int component = rows.component_id[row];
+    const float freq = (float)q.frequency_hz;
+    const double k_d = q.frequency_hz * kTwoPi / kC0;
+    PathRecord rec{};
+    bool ok = true;
+    if (component == kCidRefl) {
+        const int c = rows.primitive_id[row];
+        int d = 1;
+        while (d < kMaxDepth && c >= q.chain_offset[ends.t * kMaxDepth + d]) ++d;
+        switch (d) {
+            case 1: ok = export_chain<1>(s, q, ends, c, freq, k_d, rec); break;
+            case 2: ok = export_chain<2>(s, q, ends, c, freq, k_d, rec); break;
+            case 3: ok = export_chain<3>(s, q, ends, c, freq, k_d, rec); break;
+            case 4: ok = export_chain<4>(s, q, ends, c, freq, k_d, rec); break;
+            default: ok = export_chain<5>(s, q, ends, c, freq, k_d, rec); break;
+        }
+        if (!ok) {
+            rec.component = kCidRefl;
+            rec.depth = d;
+        }
+    } else {
+        const V3<float> seg = ends.rx - ends.tx;
+        const double dist_d = norm(to_d(ends.rx) - to_d(ends.tx));
+        const V3<float> dir = safe_normalize(seg, v3c<float>(0.f, 0.f, 1.f));
+        if (component == kCidLos) {
+            los_record(dir, ends.tx_pol, ends.rx_pol, ends.sqrt_power, (float)k_d, k_d, dist_d, rec);
+        } else {
+            // the walls are gathered again (a few rows per cell block) rather than kept per cell
+            Hit hits[kMaxHits];
+            const int d = rows.primitive_id[row];
+            straight_hits(s, q.components, q.max_depth, ends.tx, seg, dist_d, hits);
+            transmission_record<true>(s, d, hits, ends.tx, seg, dir, ends.tx_pol, ends.rx_pol, ends.sqrt_power, freq,
+                                      k_d, dist_d, rec);
+        }
+    }
+    if (!ok) rec.length = NAN;
+    write_row(rows, row, ends.t, ends.rx_id, rec);
+}
+
 // ------------------------------------------------------------------ chain cones
 __global__ void chain_cone_kernel(SceneView s, const int* __restrict__ hull_offset,
                                   const double* __restrict__ hull_points, const int* __restrict__ groups,
@@ -2270,6 +2557,84 @@ extern "C" int wc_paths_emit(const wc_scene* scene, const wc_solve* solve, const
                        *solve, row_offset, path_count, *rows);
     const hipError_t err = hipGetLastError();
     return err == hipSuccess ? 0 : wc_fail_hip("wc_paths_emit", err);
+}
+
+// Bytes of the masked export's workspace: the radiomap's up to (not with) its
+// staged diffraction records; the straight-segment codes take the place of the
+// partial sums.
+extern "C" size_t wc_paths_masks_workspace_bytes(int cells, int lanes_per_cell, int edge_count, int max_tx_chains,
+                                                 int tx_count) {
+    const int c = cells > 0 ? cells : 0;
+    return stage_base(c, lanes_per_cell > 0 ? lanes_per_cell : 1, edge_count > 0 ? edge_count : 0, max_tx_chains,
+                      tx_count) + 256;
+}
+
+static int check_masked(const wc_scene* scene, const wc_solve* q, const void* workspace, const int* tiles,
+                        int tile_count, const char* who) {
+    if (int rc = check_scene(scene)) return rc;
+    if (int rc = check_solve(q)) return rc;
+    const int width = q->lanes_per_cell;
+    if (width < 1 || width > 64 || (width & (width - 1)) != 0)
+        return wc_fail("%s: lanes_per_cell must be a power of two in [1, 64]", who);
+    if (q->total_cells == 0) return 0;
+    if (!workspace || !tiles || tile_count <= 0) return wc_fail("%s: workspace and tiles are required", who);
+    if ((size_t)tile_count > tile_capacity(q->total_cells, width, q->tx_count))
+        return wc_fail("%s: tile_count %d exceeds ceil(total_cells * lanes_per_cell / 64) + tx_count", who, tile_count);
+    return 0;
+}
+
+static const unsigned* export_diff_masks(const wc_scene* scene, const wc_solve* q, void* workspace) {
+    if (!(q->components & kCompDiff) || q->max_depth < 1 || scene->edge_count <= 0) return nullptr;
+    return reinterpret_cast<const unsigned*>(static_cast<char*>(workspace) +
+                                             partial_bytes(q->total_cells, q->lanes_per_cell));
+}
+
+extern "C" int wc_paths_count_masked(const wc_scene* scene, const wc_solve* solve, void* workspace, const int* tiles,
+                                     int tile_count, int* path_count, void* stream) {
+    if (int rc = check_masked(scene, solve, workspace, tiles, tile_count, "wc_paths_count_masked")) return rc;
+    if (solve->total_cells == 0) return 0;
+    if (!path_count) return wc_fail("wc_paths_count_masked: path_count is null");
+    const SceneView s = *reinterpret_cast<const SceneView*>(scene);
+    hipStream_t st = (hipStream_t)stream;
+    (void)hipGetLastError();
+    t_launch_error = hipSuccess;
+    wc_radiomap_out o{};
+    o.workspace = workspace;
+    const unsigned* diff = export_diff_masks(scene, solve, workspace);
+    launch_chain_visibility(s, *solve, o, tiles, tile_count, st);
+    if (diff) launch_diff_visibility(s, *solve, o, st);
+    WC_LAUNCH(export_count_kernel, dim3((tile_count + 3) / 4), dim3(256), 0, st, s, *solve, tiles, tile_count,
+              workspace, diff, path_count);
+    const hipError_t err = t_launch_error;
+    t_launch_error = hipSuccess;
+    return err == hipSuccess ? 0 : wc_fail_hip("wc_paths_count_masked", err);
+}
+
+extern "C" int wc_paths_emit_masked(const wc_scene* scene, const wc_solve* solve, void* workspace, const int* tiles,
+                                    int tile_count, const int* row_offset, const int* path_count, int total,
+                                    int* row_list, const wc_path_rows* rows, void* stream) {
+    if (int rc = check_masked(scene, solve, workspace, tiles, tile_count, "wc_paths_emit_masked")) return rc;
+    if (total < 0) return wc_fail("wc_paths_emit_masked: total must be non-negative");
+    if (!rows || !row_offset || !path_count || !row_list)
+        return wc_fail("wc_paths_emit_masked: rows / row_offset / path_count / row_list are null");
+    if (rows->width < 1 || rows->width < solve->max_depth)
+        return wc_fail("wc_paths_emit_masked: width must be >= max_depth");
+    if (solve->total_cells == 0 || total == 0) return 0;
+    const SceneView s = *reinterpret_cast<const SceneView*>(scene);
+    hipStream_t st = (hipStream_t)stream;
+    (void)hipGetLastError();
+    t_launch_error = hipSuccess;
+    int* dealt = row_list + total;  // the two lists' lengths
+    const unsigned* diff = export_diff_masks(scene, solve, workspace);
+    const unsigned blocks = (unsigned)(((long long)total + 255) / 256);
+    WC_LAUNCH(zero_int_kernel, dim3(1), dim3(64), 0, st, dealt, 2);
+    WC_LAUNCH(export_deal_kernel, dim3((tile_count + 3) / 4), dim3(256), 0, st, s, *solve, tiles, tile_count,
+              workspace, diff, row_offset, path_count, *rows, total, row_list, dealt);
+    if (diff) WC_LAUNCH(export_diff_kernel, dim3(blocks), dim3(256), 0, st, s, *solve, *rows, row_list, dealt);
+    WC_LAUNCH(export_main_kernel, dim3(blocks), dim3(256), 0, st, s, *solve, *rows, total, row_list, dealt);
+    const hipError_t err = t_launch_error;
+    t_launch_error = hipSuccess;
+    return err == hipSuccess ? 0 : wc_fail_hip("wc_paths_emit_masked", err);
 }
 
 extern "C" int wc_chain_cones(const wc_scene* scene, const int* hull_offset, const double* hull_points,

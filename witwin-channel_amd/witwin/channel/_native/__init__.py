@@ -220,6 +220,11 @@ _SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "wc_paths_count": (c_int, [ctypes.POINTER(WcScene), ctypes.POINTER(WcSolve), c_void_p, c_void_p]),
     "wc_paths_emit": (c_int, [ctypes.POINTER(WcScene), ctypes.POINTER(WcSolve), c_void_p, c_void_p,
                               ctypes.POINTER(WcPathRows), c_void_p]),
+    "wc_paths_masks_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
+    "wc_paths_count_masked": (c_int, [ctypes.POINTER(WcScene), ctypes.POINTER(WcSolve), c_void_p, c_void_p, c_int,
+                                      c_void_p, c_void_p]),
+    "wc_paths_emit_masked": (c_int, [ctypes.POINTER(WcScene), ctypes.POINTER(WcSolve), c_void_p, c_void_p, c_int,
+                                     c_void_p, c_void_p, c_int, c_void_p, ctypes.POINTER(WcPathRows), c_void_p]),
     "wc_paths_canonical_order": (c_int, [ctypes.POINTER(WcPathRows), c_void_p, c_int, c_void_p, c_void_p,
                                          c_void_p]),
     "wc_paths_compact_workspace_bytes": (c_size_t, [c_int]),

@@ -67,6 +67,38 @@ def test_cfr_kernel_matches_float64(device, mode):
     assert np.all(got[3] == 0)
 
 
+@pytest.mark.parametrize("paths, subcarriers", [(1, 2), (63, 31), (64, 33), (65, 1024), (130, 1025), (7, 992)])
+def test_cfr_grid_tiles(device, paths, subcarriers):
+    """Uniform grids at the edges of the 64-path chunks and of the 32 x 32
+    subcarrier blocks. The row and column phasors are each rounded once where
+    one phasor was before: 2e-6 of sum |a| stays the bound."""
+    _say(f"case: CFR grid, {paths} paths, {subcarriers} subcarriers")
+    rng = np.random.default_rng(paths)
+    b = 5
+    a = (rng.normal(size=(b, paths, 1)) + 1j * rng.normal(size=(b, paths, 1))).astype(np.complex64)
+    tau = rng.uniform(1e-7, 3e-6, (b, paths)).astype(np.float32)
+    valid = rng.uniform(size=(b, paths)) < 0.8
+    valid[0] = True
+    freqs = 3.5e9 + 30e3 * np.arange(subcarriers)
+    got = path.paths_cfr(torch.as_tensor(a).to(device), torch.as_tensor(tau).to(device),
+                         torch.as_tensor(valid).to(device), torch.as_tensor(freqs)).cpu().numpy()
+    ref = _cfr_float64(a, tau, valid, freqs, True)
+    assert (np.abs(got - ref) / (np.abs(a).sum(axis=1)[:, :, None] + 1e-30)).max() <= 2e-6
+
+
+def test_cfr_grid_infinite_amplitude(device):
+    """An infinite part spreads as in the sum of products, not as NaN."""
+    a = torch.tensor([[[1.0 + 1.0j], [complex(float("inf"), 0.0)]]], dtype=torch.complex64, device=device)
+    tau = torch.tensor([[1.0e-6, 1.3e-6]], device=device)
+    valid = torch.ones((1, 2), dtype=torch.bool, device=device)
+    freqs = torch.as_tensor(28.0e9 + 1.0e5 * np.arange(40))
+    grid = path.paths_cfr(a, tau, valid, freqs, normalize_delays=False)
+    listed = path.paths_cfr(a, tau, valid, freqs.to(device), normalize_delays=False)
+    assert torch.equal(torch.view_as_real(grid).nan_to_num(7.0, 8.0, 9.0) > 6.0,
+                       torch.view_as_real(listed).nan_to_num(7.0, 8.0, 9.0) > 6.0)
+    assert bool(torch.isinf(grid.real).all())
+
+
 def test_cfr_kernel_empty_inputs(device):
     out = path.paths_cfr(torch.zeros((4, 0, 1), dtype=torch.complex64, device=device),
                          torch.zeros((4, 0), device=device), torch.zeros((4, 0), dtype=torch.bool, device=device),

@@ -261,7 +261,8 @@ def paths_cfr(a: torch.Tensor, tau: torch.Tensor, valid: torch.Tensor, frequenci
     f0, df = grid if grid is not None else (0.0, 0.0)
     a_c = a.contiguous()
     tau_c = tau.to(torch.float32).contiguous()
-    valid_c = valid.to(torch.uint8).contiguous()
+    valid_c = valid.contiguous()
+    valid_c = valid_c.view(torch.uint8) if valid_c.dtype == torch.bool else valid_c.to(torch.uint8)
     p_ = _native.ptr
     _native.call("wc_paths_cfr", p_(torch.view_as_real(a_c)) if a_c.numel() else None, p_(tau_c), p_(valid_c), b, p,
                  s, p_(freq_dev), ctypes.c_double(f0), ctypes.c_double(df), f_count, 1 if normalize_delays else 0,

@@ -10,6 +10,7 @@
 // by rows (the frequency, layer tables) get their gradients from per-row
 // partials reduced on the device.
 #include "wc_api_internal.h"
+#include "wc_adjoint.h"
 #include "wc_paths.h"
 #include "wc_tangent.h"
 #include "../../include/wcmi.h"
@@ -199,6 +200,11 @@ __device__ __forceinline__ V3<float> ld3o(const float* p, size_t i) {
     return p ? ld3(p + 3 * i) : v3c<float>(0.f, 0.f, 0.f);
 }
 __device__ __forceinline__ float ldo(const float* p, size_t i) { return p ? p[i] : 0.0f; }
+__device__ __forceinline__ void st3(float* p, const V3<float>& v) {
+    p[0] = v.x;
+    p[1] = v.y;
+    p[2] = v.z;
+}
 
 // Output views and cotangents of the shared enumerated-field schema.
 struct FieldOutPtrs {
@@ -358,55 +364,159 @@ struct ReflGrads {
     float *src, *tgt, *pos, *nrm, *eps, *sig, *gain, *thick, *freq_row;
 };
 
+// Adjoint of one row, forward values first and one reverse sweep over the
+// bounces (D is a compile-time constant, so the per-bounce fields, directions
+// and fallbacks stay in registers: D = 3 takes no private memory). Where every
+// cotangent of the field outputs is zero the field is not differentiated, so
+// rows a program masks out by zero cotangents give zeros whatever they hold.
+// ALU and launch bound: with Dual<8> passes over the 7 + 10 D input scalars
+// (37 at D = 3: five evaluations of nine numbers per scalar, in private
+// memory) 262,144 rows of three bounces took 1,324 us, the sweep takes 66; error
+// against 64 bits 6.0e-5 then, 4.2e-5 now.
+template <int D>
 __global__ void __launch_bounds__(128) refl_vjp_kernel(int n, ReflIn in, double freq, FieldGrads g, ReflGrads out) {
-    const int D = in.depth;
-    const int slots = 7 + 10 * D;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += blockDim.x * gridDim.x) {
-        float fr = 0.0f;
-        for (int pass = 0; pass * 8 < slots; ++pass) {
-            auto v3 = [&](const float* p, size_t k, int s0) {
-                const V3<float> a = ld3(p + 3 * k);
-                return V3<R8>{sv(a.x, s0, pass), sv(a.y, s0 + 1, pass), sv(a.z, s0 + 2, pass)};
-            };
-            V3<R8> pos[kMaxDepth], nrm[kMaxDepth];
-            R8 eps[kMaxDepth], sig[kMaxDepth], gain[kMaxDepth], thick[kMaxDepth];
-            float mu[kMaxDepth];
+        const V3<float> ez{0.f, 0.f, 1.f};
+        const V3<float> src = ld3(in.src + 3 * (size_t)i), tgt = ld3(in.tgt + 3 * (size_t)i);
+        const V3<float> txp = ld3(in.txp + 3 * (size_t)i), rxp = ld3(in.rxp + 3 * (size_t)i);
+        const float sp = sqrtf(fmaxf(in.power[i], 0.0f));
+        const float f = (float)freq;
+        V3<float> pos[D], nrm[D], inc[D], fall[D];  // fall: fallback of the incident direction
+        C3<float> val_in[D];
+        float seg_len[D + 1];
+        float total = 0.0f;
+        double total_d = 0.0;
+        V3<float> prev = src;
+#pragma unroll
+        for (int b = 0; b < D; ++b) {
+            pos[b] = ld3(in.pos + 3 * ((size_t)i * D + b));
+            nrm[b] = ld3(in.nrm + 3 * ((size_t)i * D + b));
+        }
+        const V3<float> first = safe_normalize(pos[0] - src, ez);
+        C3<float> value = c3_from_real(transverse(first, txp));
+        V3<float> outgoing = first;
+#pragma unroll
+        for (int b = 0; b < D; ++b) {
+            const size_t k = (size_t)i * D + b;
+            fall[b] = outgoing;
+            const V3<float> seg = pos[b] - prev;
+            inc[b] = safe_normalize(seg, outgoing);
+            seg_len[b] = norm(seg);
+            total += seg_len[b];
+            total_d += norm(to_d(pos[b]) - to_d(prev));
+            val_in[b] = value;
+            value = reflect_c3(value, inc[b], nrm[b], in.eps[k], in.sig[k], in.mu[k], in.gain[k], in.thick[k], f,
+                               outgoing);
+            prev = pos[b];
+        }
+        const V3<float> last = tgt - prev;
+        const V3<float> dir = safe_normalize(last, outgoing);
+        seg_len[D] = norm(last);
+        total += seg_len[D];
+        total_d += norm(to_d(tgt) - to_d(prev));
+        const double k_d = freq * kTwoPi / kC0;
+        const float kw = wave_number(f);
+        const float ka = fmaxf(kw, kSmallEpsF), la = fmaxf(total, kEpsF);
+        const Cx<float> prop = scale(cexpj(neg_kd_phase(k_d, total_d)), 1.0f / (ka * la * 2.0f));
+
+        // cotangents of the outputs
+        auto ldc = [&](const float* p, size_t j) { return p ? Cx<float>{p[2 * j], p[2 * j + 1]} : Cx<float>{0.f, 0.f}; };
+        C3<float> g_field{ldc(g.field_vector, 3 * (size_t)i), ldc(g.field_vector, 3 * (size_t)i + 1),
+                          ldc(g.field_vector, 3 * (size_t)i + 2)};
+        const Cx<float> gc = ldc(g.coefficient, i), gp = ldc(g.path_field, i);
+        const float gg = g.path_gain ? g.path_gain[i] : 0.0f;
+        V3<float> g_dir = ld3o(g.direction, i);
+        float g_total = ldo(g.path_length, i) + ldo(g.delay, i) * (float)(1.0 / kC0);
+        float g_freq = 0.0f;
+        auto some = [](const Cx<float>& c) { return c.re != 0.0f || c.im != 0.0f; };
+        const bool live = some(g_field.x) || some(g_field.y) || some(g_field.z) || some(gc) || some(gp) || gg != 0.0f;
+
+        if (!live && g_total == 0.0f && g_dir.x == 0.0f && g_dir.y == 0.0f && g_dir.z == 0.0f) {
+            if (out.src) st3(out.src + 3 * (size_t)i, zero3());
+            if (out.tgt) st3(out.tgt + 3 * (size_t)i, zero3());
             for (int b = 0; b < D; ++b) {
                 const size_t k = (size_t)i * D + b;
-                const int s = 7 + 10 * b;
-                pos[b] = v3(in.pos, k, s);
-                nrm[b] = v3(in.nrm, k, s + 3);
-                eps[b] = sv(in.eps[k], s + 6, pass);
-                sig[b] = sv(in.sig[k], s + 7, pass);
-                gain[b] = sv(in.gain[k], s + 8, pass);
-                thick[b] = sv(in.thick[k], s + 9, pass);
-                mu[b] = in.mu[k];
+                if (out.pos) st3(out.pos + 3 * k, zero3());
+                if (out.nrm) st3(out.nrm + 3 * k, zero3());
+                if (out.eps) out.eps[k] = 0.0f;
+                if (out.sig) out.sig[k] = 0.0f;
+                if (out.gain) out.gain[k] = 0.0f;
+                if (out.thick) out.thick[k] = 0.0f;
             }
-            RowOut<R8> r;
-            reflection_row<R8>(D, v3(in.src, i, 0), v3(in.tgt, i, 3), pos, nrm, eps, sig, mu, gain, thick,
-                               ld3(in.txp + 3 * i), ld3(in.rxp + 3 * i), sqrtf(fmaxf(in.power[i], 0.0f)),
-                               sv((float)freq, 6, pass), freq, r);
-            float d[8];
-            contract_row(g, i, r, d);
-            for (int j = 0; j < 8; ++j) {
-                const int s = 8 * pass + j;
-                if (s >= slots) break;
-                if (s < 3) { if (out.src) out.src[3 * i + s] = d[j]; }
-                else if (s < 6) { if (out.tgt) out.tgt[3 * i + s - 3] = d[j]; }
-                else if (s == 6) fr = d[j];
-                else {
-                    const int b = (s - 7) / 10, q = (s - 7) % 10;
-                    const size_t k = (size_t)i * D + b;
-                    if (q < 3) { if (out.pos) out.pos[3 * k + q] = d[j]; }
-                    else if (q < 6) { if (out.nrm) out.nrm[3 * k + q - 3] = d[j]; }
-                    else if (q == 6) { if (out.eps) out.eps[k] = d[j]; }
-                    else if (q == 7) { if (out.sig) out.sig[k] = d[j]; }
-                    else if (q == 8) { if (out.gain) out.gain[k] = d[j]; }
-                    else { if (out.thick) out.thick[k] = d[j]; }
-                }
-            }
+            out.freq_row[i] = 0.0f;
+            continue;
         }
-        out.freq_row[i] = fr;
+
+        V3<float> g_pos_next = zero3();  // cotangent of the point the sweep stands at
+        V3<float> g_out = zero3();       // of the direction leaving bounce b
+        C3<float> g_value{{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
+        if (live) {
+            const C3<float> field = c3_scale(value, prop);
+            const V3<float> tr = transverse(dir, rxp);
+            const Cx<float> pf = scale(c3_dot_real(field, tr), sp);
+            const Cx<float> g_pf{gp.re + 2.0f * gg * pf.re, gp.im + 2.0f * gg * pf.im};
+            const Cx<float> g_coef{gc.re + sp * g_pf.re, gc.im + sp * g_pf.im};
+            const V3<float> g_tr = c3_axis_adj(field, g_coef);
+            V3<float> none = zero3();
+            transverse_adj(dir, rxp, g_tr, g_dir, none);
+            g_field = g_field + c3_axis(tr, g_coef);
+            const Cx<float> g_prop = cmulj(value.x, g_field.x) + cmulj(value.y, g_field.y) + cmulj(value.z, g_field.z);
+            g_value = {cmulj(prop, g_field.x), cmulj(prop, g_field.y), cmulj(prop, g_field.z)};
+            float g_k = 0.0f;
+            carrier_adj(prop, kw, ka, total, la, kw >= kSmallEpsF, total >= kEpsF, g_prop, g_k, g_total, g_total);
+            g_freq += g_k * (float)(kTwoPi / kC0);
+        }
+        V3<float> g_tgt = zero3();
+        {
+            V3<float> g_seg = zero3();
+            safe_normalize_adj(last, outgoing, g_dir, g_seg, g_out);
+            norm_adj(last, seg_len[D], g_total, g_seg);
+            g_tgt = g_seg;
+            g_pos_next = -g_seg;
+        }
+#pragma unroll
+        for (int b = D - 1; b >= 0; --b) {
+            const size_t k = (size_t)i * D + b;
+            V3<float> g_inc = zero3(), g_nrm = zero3();
+            SlabGrad sg{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            // the reflected direction matters to the field and, as a fallback, to later directions
+            const bool turned = g_out.x != 0.0f || g_out.y != 0.0f || g_out.z != 0.0f;
+            if (live || turned) {
+                C3<float> g_in;
+                reflect_c3_adj(val_in[b], inc[b], nrm[b], in.eps[k], in.sig[k], in.mu[k], in.gain[k], in.thick[k], f,
+                               g_value, g_out, g_in, g_inc, g_nrm, sg);
+                g_value = g_in;
+            }
+            g_freq += sg.freq;
+            if (out.nrm) st3(out.nrm + 3 * k, g_nrm);
+            if (out.eps) out.eps[k] = sg.eps;
+            if (out.sig) out.sig[k] = sg.sig;
+            if (out.gain) out.gain[k] = sg.gain;
+            if (out.thick) out.thick[k] = sg.thick;
+            if (b == 0) {
+                // the launch polarization is transverse to the first direction
+                const V3<float> g_t{g_value.x.re, g_value.y.re, g_value.z.re};
+                V3<float> g_first = zero3(), none = zero3();
+                transverse_adj(first, txp, g_t, g_first, none);
+                g_out = g_first;
+            } else {
+                g_out = zero3();
+            }
+            const V3<float> seg = pos[b] - (b ? pos[b ? b - 1 : 0] : src);
+            V3<float> g_seg = zero3();
+            safe_normalize_adj(seg, fall[b], g_inc, g_seg, g_out);
+            if (b == 0) {
+                V3<float> none = zero3();
+                safe_normalize_adj(seg, ez, g_out, g_seg, none);
+            }
+            norm_adj(seg, seg_len[b], g_total, g_seg);
+            const V3<float> g_p = g_pos_next + g_seg;
+            if (out.pos) st3(out.pos + 3 * k, g_p);
+            g_pos_next = -g_seg;
+        }
+        if (out.src) st3(out.src + 3 * (size_t)i, g_pos_next);
+        if (out.tgt) st3(out.tgt + 3 * (size_t)i, g_tgt);
+        out.freq_row[i] = g_freq;
     }
 }
 
@@ -697,18 +807,47 @@ __global__ void __launch_bounds__(128) stack_vjp_kernel(int n, StackIn in, doubl
 }
 
 // ------------------------------------------------------------------ reductions
-// sum of n floats in a fixed order (one block): strided float64 partials, tree
-__global__ void __launch_bounds__(256) sum_rows_kernel(const float* __restrict__ x, int n, float* __restrict__ out) {
+// Sum of n floats in a fixed order, float64. Up to kSumChunk one workgroup does
+// it all. Beyond, one workgroup per chunk leaves its sum in the chunk's own
+// first eight bytes (its floats are read by then) and one more adds those: a
+// single workgroup walks 262,144 floats in 255 us, the two launches in 10.
+constexpr int kSumChunk = 4096;
+
+__device__ __forceinline__ double block_sum(double acc) {
     __shared__ double part[256];
-    double acc = 0.0;
-    for (int i = threadIdx.x; i < n; i += 256) acc += (double)x[i];
     part[threadIdx.x] = acc;
     __syncthreads();
     for (int h = 128; h > 0; h >>= 1) {
         if ((int)threadIdx.x < h) part[threadIdx.x] += part[threadIdx.x + h];
         __syncthreads();
     }
-    if (threadIdx.x == 0) *out = (float)part[0];
+    return part[0];
+}
+
+__global__ void __launch_bounds__(256) sum_rows_kernel(const float* __restrict__ x, int n, float* __restrict__ out) {
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < n; i += 256) acc += (double)x[i];
+    acc = block_sum(acc);
+    if (threadIdx.x == 0) *out = (float)acc;
+}
+
+// chunk c: x[c kSumChunk ..), the last one with the remainder too, so every
+// chunk holds at least two floats; the sum goes to the first two (8-byte
+// aligned: the workspace is, and kSumChunk is even)
+__global__ void __launch_bounds__(256) sum_chunks_kernel(float* x, int n) {
+    const size_t base = (size_t)blockIdx.x * kSumChunk;
+    const int count = (int)blockIdx.x + 1 < (int)gridDim.x ? kSumChunk : n - (int)base;
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < count; i += 256) acc += (double)x[base + i];
+    acc = block_sum(acc);
+    if (threadIdx.x == 0) *reinterpret_cast<double*>(x + base) = acc;
+}
+
+__global__ void __launch_bounds__(256) sum_partials_kernel(const float* x, int chunks, float* __restrict__ out) {
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < chunks; i += 256) acc += *reinterpret_cast<const double*>(x + (size_t)i * kSumChunk);
+    acc = block_sum(acc);
+    if (threadIdx.x == 0) *out = (float)acc;
 }
 
 __global__ void cast_layers_kernel(const double* __restrict__ acc, int n, float* __restrict__ out) {
@@ -720,6 +859,17 @@ __global__ void zero_doubles_kernel(double* p, int n) {
 }
 
 int row_blocks(int n) { return std::max(1, std::min((n + 127) / 128, 65536)); }
+
+// sum of the workspace's n per-row partials (overwritten)
+void sum_rows(float* rows, int n, float* out, hipStream_t st) {
+    const int chunks = n / kSumChunk;
+    if (chunks <= 1) {
+        hipLaunchKernelGGL(sum_rows_kernel, dim3(1), dim3(256), 0, st, rows, n, out);
+        return;
+    }
+    hipLaunchKernelGGL(sum_chunks_kernel, dim3(chunks), dim3(256), 0, st, rows, n);
+    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, st, rows, chunks, out);
+}
 
 FieldOutPtrs out_ptrs(const wc_field_rows_out* o) {
     return {o->field_vector, o->coefficient, o->path_field, o->path_gain, o->path_length_m, o->delay_s, o->direction};
@@ -808,7 +958,7 @@ extern "C" int wc_field_free_space_vjp(int count, const float* source, const flo
         hipLaunchKernelGGL(fs_vjp_kernel, dim3(row_blocks(count)), dim3(128), 0, st, count, source, target, tx_power,
                            tx_polarization, rx_polarization, frequency_hz, grad_ptrs(grads), grad_source, grad_target,
                            v.freq_row);
-    hipLaunchKernelGGL(sum_rows_kernel, dim3(1), dim3(256), 0, st, v.freq_row, count, grad_frequency);
+    sum_rows(v.freq_row, count, grad_frequency, st);
     const hipError_t err = hipGetLastError();
     return err == hipSuccess ? 0 : wc_fail_hip(who, err);
 }
@@ -855,10 +1005,16 @@ extern "C" int wc_field_reflection_sequence_vjp(const wc_reflection_rows* rows, 
     const ReflGrads g{out->grad_source, out->grad_target, out->grad_interaction_positions,
                       out->grad_interaction_normals, out->grad_eps_r, out->grad_sigma_e, out->grad_gain,
                       out->grad_thickness, v.freq_row};
-    if (rows->count > 0)
-        hipLaunchKernelGGL(refl_vjp_kernel, dim3(row_blocks(rows->count)), dim3(128), 0, st, rows->count,
-                           refl_in(rows), rows->frequency_hz, grad_ptrs(grads), g);
-    hipLaunchKernelGGL(sum_rows_kernel, dim3(1), dim3(256), 0, st, v.freq_row, rows->count, out->grad_frequency);
+    if (rows->count > 0) {
+        auto* kernel = rows->depth == 1   ? refl_vjp_kernel<1>
+                       : rows->depth == 2 ? refl_vjp_kernel<2>
+                       : rows->depth == 3 ? refl_vjp_kernel<3>
+                       : rows->depth == 4 ? refl_vjp_kernel<4>
+                                          : refl_vjp_kernel<5>;
+        hipLaunchKernelGGL(kernel, dim3(row_blocks(rows->count)), dim3(128), 0, st, rows->count, refl_in(rows),
+                           rows->frequency_hz, grad_ptrs(grads), g);
+    }
+    sum_rows(v.freq_row, rows->count, out->grad_frequency, st);
     const hipError_t err = hipGetLastError();
     return err == hipSuccess ? 0 : wc_fail_hip(who, err);
 }
@@ -940,7 +1096,7 @@ extern "C" int wc_field_transmission_sequence_vjp(const wc_transmission_rows* ro
     if (rows->count > 0)
         hipLaunchKernelGGL(trans_vjp_kernel, dim3(row_blocks(rows->count)), dim3(128), 0, st, rows->count,
                            trans_in(rows), rows->frequency_hz, grad_ptrs(grads), g);
-    hipLaunchKernelGGL(sum_rows_kernel, dim3(1), dim3(256), 0, st, v.freq_row, rows->count, grad_frequency);
+    sum_rows(v.freq_row, rows->count, grad_frequency, st);
     if (layers > 0) {
         const int b = std::max(1, (layers + 255) / 256);
         if (grad_layer_thickness) hipLaunchKernelGGL(cast_layers_kernel, dim3(b), dim3(256), 0, st, v.thick, layers,
@@ -1027,7 +1183,7 @@ extern "C" int wc_em_layer_stack_vjp(int count, const float* cos_theta, const in
     if (count > 0)
         hipLaunchKernelGGL(stack_vjp_kernel, dim3(row_blocks(count)), dim3(128), 0, st, count, in, frequency_hz, g,
                            grad_cos_theta, v.freq_row, v.thick, v.eps, v.sig);
-    hipLaunchKernelGGL(sum_rows_kernel, dim3(1), dim3(256), 0, st, v.freq_row, count, grad_frequency);
+    sum_rows(v.freq_row, count, grad_frequency, st);
     if (nl > 0) {
         const int b = std::max(1, (nl + 255) / 256);
         if (grad_layer_thickness)

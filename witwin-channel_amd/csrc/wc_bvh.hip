@@ -110,31 +110,36 @@ __global__ void radix_histogram_kernel(const unsigned int* __restrict__ keys, in
     for (int d = threadIdx.x; d < kRadix; d += blockDim.x) hist[d * blocks + blockIdx.x] = counts[d];
 }
 
-// exclusive scan of hist (digit-major, block-minor) in one workgroup
-__global__ void radix_scan_kernel(int* __restrict__ hist, int count) {
-    __shared__ int partial[1024];
-    const int tid = threadIdx.x;
-    const int per = (count + blockDim.x - 1) / blockDim.x;
-    const int begin = tid * per;
-    const int end = min(begin + per, count);
-    int sum = 0;
-    for (int i = begin; i < end; ++i) sum += hist[i];
-    partial[tid] = sum;
-    __syncthreads();
-    if (tid == 0) {
-        int run = 0;
-        for (int i = 0; i < (int)blockDim.x; ++i) {
-            const int v = partial[i];
-            partial[i] = run;
-            run += v;
-        }
+// Inclusive scan over a wavefront.
+__device__ __forceinline__ int wave_scan(int v, int lane) {
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(v, off);
+        if (lane >= off) v += y;
     }
-    __syncthreads();
-    int run = partial[tid];
-    for (int i = begin; i < end; ++i) {
-        const int v = hist[i];
-        hist[i] = run;
-        run += v;
+    return v;
+}
+
+// Inclusive scan of hist over the blocks of each digit (digit-major,
+// block-minor), one workgroup per digit, 256 blocks a round. The scatter adds
+// the digits' bases, the exclusive scan of the row ends, itself: the whole
+// table in one workgroup cost 66 us a pass at 64 blocks (262,144 keys) and
+// 3.7 ms at 4,096, most of a pass's time.
+__global__ void __launch_bounds__(256) radix_scan_kernel(int* __restrict__ hist, int blocks) {
+    __shared__ int wave_total[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int* row = hist + (size_t)blockIdx.x * blocks;
+    int carry = 0;
+    for (int base = 0; base < blocks; base += 256) {
+        const int i = base + tid;
+        int x = wave_scan(i < blocks ? row[i] : 0, lane);
+        if (lane == 63) wave_total[wave] = x;
+        __syncthreads();
+        int before = carry;
+        for (int w = 0; w < wave; ++w) before += wave_total[w];
+        if (i < blocks) row[i] = before + x;
+        for (int w = 0; w < 4; ++w) carry += wave_total[w];
+        __syncthreads();  // wave_total is rewritten by the next round
     }
 }
 
@@ -150,7 +155,18 @@ __global__ void radix_scatter_kernel(const unsigned int* __restrict__ keys_in, c
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-    for (int d = tid; d < kRadix; d += blockDim.x) offsets[d] = hist[d * blocks + blockIdx.x];
+    // first slot of each digit: the digits before it, then the blocks before this one
+    static_assert(kSortThreads == kRadix, "one thread per digit");
+    {
+        const int total = hist[(size_t)tid * blocks + blocks - 1];
+        const int x = wave_scan(total, lane);
+        if (lane == 63) wave_counts[0][wave] = x;
+        __syncthreads();
+        int before = x - total + (blockIdx.x ? hist[(size_t)tid * blocks + blockIdx.x - 1] : 0);
+        for (int w = 0; w < wave; ++w) before += wave_counts[0][w];
+        offsets[tid] = before;
+        __syncthreads();  // wave_counts is cleared below
+    }
     const int base = blockIdx.x * kSortTile;
     const unsigned long long lane_lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
     for (int it = 0; it < kSortItems; ++it) {
@@ -361,7 +377,7 @@ int radix_sort_pairs(unsigned int* keys, int* values, unsigned int* keys_tmp, in
         const int shift = p * kRadixBits;
         hipLaunchKernelGGL(radix_histogram_kernel, dim3(blocks), dim3(kSortThreads), 0, stream, kin, n, shift, hist,
                            blocks);
-        hipLaunchKernelGGL(radix_scan_kernel, dim3(1), dim3(1024), 0, stream, hist, kRadix * blocks);
+        hipLaunchKernelGGL(radix_scan_kernel, dim3(kRadix), dim3(256), 0, stream, hist, blocks);
         hipLaunchKernelGGL(radix_scatter_kernel, dim3(blocks), dim3(kSortThreads), 0, stream, kin, vin, kout, vout, n,
                            shift, hist, blocks);
         std::swap(kin, kout);

@@ -27,6 +27,17 @@ int plan_grid(long long n) {
 constexpr int kPlanDepths = WC_PLAN_DEPTHS;
 constexpr unsigned long long kNoKey = ~0ull;
 
+// Bits that order the keys of one depth: keys are below parents * group_count,
+// and kNoKey, cut to these bits, still comes after all of them. Sorting only
+// these takes 10 passes for three depths of 262,144 rays over 386 groups where
+// both full words take 24.
+int key_bits(long long parents, int group_count) {
+    const unsigned long long keys = (unsigned long long)parents * (unsigned long long)group_count;
+    int bits = 1;
+    while (bits < 64 && (1ull << bits) - 1 < keys) ++bits;
+    return bits;
+}
+
 // key of ray i at depth d (kNoKey: no d-prefix)
 __device__ __forceinline__ unsigned long long prefix_key(const int* __restrict__ rays, const int* __restrict__ pid,
                                                          long long i, int ray_count, int max_depth, int d,
@@ -207,12 +218,16 @@ extern "C" int wc_plan_level(const int* rays, int tx_count, int ray_count, int m
                            counts, tx_count * kPlanDepths);
     hipLaunchKernelGGL(plan_keys_kernel, dim3(plan_grid(n)), dim3(256), 0, st, rays, pid, n, ray_count, max_depth, d,
                        group_count, lo, vals);
-    if (radix_sort_pairs(lo, vals, keys_tmp, vals_tmp, hist, (int)n, 32, st) != 0)
+    // parents of depth 1 are the transmitters, later ones the runs of at most n rays
+    const int bits = key_bits(d == 1 ? tx_count : n, group_count);
+    if (radix_sort_pairs(lo, vals, keys_tmp, vals_tmp, hist, (int)n, std::min(bits, 32), st) != 0)
         return wc_fail_hip("wc_plan_level: radix sort (low word)", hipGetLastError());
-    hipLaunchKernelGGL(plan_high_kernel, dim3(plan_grid(n)), dim3(256), 0, st, rays, pid, n, ray_count, max_depth, d,
-                       group_count, vals, hi);
-    if (radix_sort_pairs(hi, vals, keys_tmp, vals_tmp, hist, (int)n, 32, st) != 0)
-        return wc_fail_hip("wc_plan_level: radix sort (high word)", hipGetLastError());
+    if (bits > 32) {
+        hipLaunchKernelGGL(plan_high_kernel, dim3(plan_grid(n)), dim3(256), 0, st, rays, pid, n, ray_count, max_depth,
+                           d, group_count, vals, hi);
+        if (radix_sort_pairs(hi, vals, keys_tmp, vals_tmp, hist, (int)n, bits - 32, st) != 0)
+            return wc_fail_hip("wc_plan_level: radix sort (high word)", hipGetLastError());
+    }
     hipLaunchKernelGGL(plan_heads_kernel, dim3(plan_grid(n)), dim3(256), 0, st, rays, pid, n, ray_count, max_depth, d,
                        group_count, vals, head);
     if (scan_exclusive(head, (int)n, first, ws + l.scan, prefix_count, st) != 0)

@@ -6,9 +6,13 @@
 // over values that are not numbers. Prints "depth kind errors" per input kind:
 // the 2-norm of the difference over the 2-norm of the tangent contraction over
 // the ordinary rows and over the degenerate ones, and the number of non-zeros
-// in masked rows.
+// in masked rows. Then the stored-path sweeps of the radiomap adjoint
+// (wc_path_adjoint.h) against the dual-number evaluators (wc_tangent.h) over
+// random planes and layered walls: "planes" and "wall_normals", coherent and
+// incoherent.
 #include "hip/hip_runtime.h"
 #include "../../witwin-channel_amd/csrc/wc_rows.hip"
+#include "../../witwin-channel_amd/csrc/wc_path_adjoint.h"
 
 #include <cstdio>
 #include <random>
@@ -124,7 +128,132 @@ template <int D> static void check(int n, double freq) {
                     std::sqrt(num[1][k] / den[1][k]), nonzero);
 }
 
+// ---- stored paths of the radiomap
+struct Sum {
+    double num = 0, den = 0;
+    void add(double got, double want) {
+        num += (got - want) * (got - want);
+        den += want * want;
+    }
+    double error() const { return std::sqrt(num / den); }
+};
+
+// <cotangent, d path / d slot i> of a dual evaluation
+template <int N>
+static void contract_dual(const C3<Dual<N>>& f, const V3<Dual<N>>& dir, const V3<float>& rx_pol, const PathCotangent& w,
+                          double d[N]) {
+    const Cx<Dual<N>> c = project_receiver(f, dir, lift3<Dual<N>>(rx_pol));
+    const Cx<float> g = coefficient_cotangent(w, cval(c));
+    for (int i = 0; i < N; ++i) d[i] = (double)g.re * c.re.d[i] + (double)g.im * c.im.d[i];
+}
+
+static void check_paths(int n, double freq, bool coherent) {
+    std::mt19937 gen(coherent ? 7 : 8);
+    std::uniform_real_distribution<float> u01(0.0f, 1.0f);
+    auto uni = [&](float lo, float hi) { return lo + (hi - lo) * u01(gen); };
+    auto vec = [&](float lo, float hi) { return V3<float>{uni(lo, hi), uni(lo, hi), uni(lo, hi)}; };
+    auto unit3 = [&] {
+        V3<float> v = vec(-1, 1);
+        return v * (1.0f / norm(v));
+    };
+    constexpr int M = 6;
+    std::vector<float> eps, sig, mu, gain, thick, lt, le, ls, lm;
+    std::vector<int> lo, lc;
+    for (int m = 0; m < M; ++m) {
+        eps.push_back(uni(2, 6)); sig.push_back(uni(0.001f, 0.04f)); mu.push_back(1.0f); gain.push_back(uni(0.6f, 1));
+        thick.push_back(uni(0.02f, 0.2f));
+        lo.push_back((int)lt.size());
+        lc.push_back(1 + m % 4);
+        for (int l = 0; l < lc.back(); ++l) {
+            lt.push_back(uni(0.01f, 0.1f)); le.push_back(uni(2, 5)); ls.push_back(uni(0.001f, 0.03f)); lm.push_back(1.0f);
+        }
+    }
+    constexpr int G = 40;
+    std::vector<double> plane;
+    std::vector<int> fmat;
+    for (int g = 0; g < G; ++g) {
+        const V3<float> v = unit3();
+        plane.insert(plane.end(), {(double)v.x, (double)v.y, (double)v.z, (double)uni(-40, 40)});
+        fmat.push_back(g % M);
+    }
+    SceneView s{};
+    s.group_plane = plane.data(); s.face_material = fmat.data();
+    s.mat_eps = eps.data(); s.mat_sigma = sig.data(); s.mat_mu = mu.data(); s.mat_gain = gain.data();
+    s.mat_thickness = thick.data(); s.mat_layer_offset = lo.data(); s.mat_layer_count = lc.data();
+    s.layer_thickness = lt.data(); s.layer_eps = le.data(); s.layer_sigma = ls.data(); s.layer_mu = lm.data();
+    s.material_count = M;
+    const double k_d = freq * kTwoPi / kC0;
+    const float f = (float)freq;
+    constexpr int DM = kMaxDepth;
+    Sum planes, wall_n;
+    for (int i = 0; i < n; ++i) {
+        PathCotangent w;
+        w.coherent = coherent;
+        w.sp = uni(0.5f, 1.5f);
+        w.a = {uni(-1, 1), uni(-1, 1)};
+        w.inc = uni(-1, 1);
+        const V3<float> tx = vec(0, 60), rx = vec(0, 60), txp = unit3(), rxp = unit3();
+        const int depth = 1 + i % DM;
+        int groups[DM], mats[DM];
+        Hit hits[kMaxHits];
+        for (int b = 0; b < DM; ++b) {
+            groups[b] = (int)(gen() % G);
+            if (b && groups[b] == groups[b - 1]) groups[b] = (groups[b] + 1) % G;
+            mats[b] = fmat[groups[b]];
+            hits[b] = {0.0f, groups[b], groups[b]};
+        }
+        // unfolded length in double, as the forward pass has it
+        V3<double> p = to_d(tx);
+        for (int b = 0; b < depth; ++b) {
+            double o;
+            const V3<double> nv = group_normal(s, groups[b], o);
+            p = p - nv * (2.0 * (dot(p, nv) - o));
+        }
+        const double length = norm(to_d(rx) - p), dist = norm(to_d(rx) - to_d(tx));
+        using D1 = Dual<1>;
+        auto sd = [](float v, bool on) {
+            D1 r = make_dual<1>(v);
+            r.d[0] = on ? 1.0f : 0.0f;
+            return r;
+        };
+        PlaneGrad<DM> bp, bn;
+        reflection_planes<DM>(s, depth, groups, mats, tx, rx, txp, rxp, f, k_d, length, w, bp);
+        const int nw = i % (DM + 1);
+        straight_normals<DM>(s, nw, hits, tx, rx, txp, rxp, f, k_d, dist, w, bn);
+        for (int slot = 0; slot < 4 * DM; ++slot) {
+            V3<D1> nv[DM];
+            D1 off[DM];
+            for (int b = 0; b < DM; ++b) {
+                double o;
+                const V3<float> v = to_f(group_normal(s, groups[b], o));
+                nv[b] = {sd(v.x, slot == 4 * b), sd(v.y, slot == 4 * b + 1), sd(v.z, slot == 4 * b + 2)};
+                off[b] = sd((float)o, slot == 4 * b + 3);
+            }
+            const int b = slot / 4, c = slot % 4;
+            auto value = [&](const PlaneGrad<DM>& o) {
+                return c == 0 ? o.nrm[b].x : c == 1 ? o.nrm[b].y : c == 2 ? o.nrm[b].z : o.off[b];
+            };
+            V3<D1> dir;
+            double d[1];
+            if (b < depth) {
+                contract_dual<1>(reflection_tangent_planes(s, depth, groups, nv, off, tx, rx, txp, f, k_d, length, dir),
+                                 dir, rxp, w, d);
+                planes.add(value(bp), d[0]);
+            }
+            if (b < nw && c < 3) {
+                contract_dual<1>(transmission_tangent_walls(s, nw, hits, nv, tx, rx, txp, f, k_d, dist, dir), dir, rxp,
+                                 w, d);
+                wall_n.add(value(bn), d[0]);
+            }
+        }
+    }
+    const char* mode = coherent ? "coherent" : "incoherent";
+    std::printf("%s planes %.3e\n%s wall_normals %.3e\n", mode, planes.error(), mode, wall_n.error());
+}
+
 int main() {
+    check_paths(4000, 3.5e9, true);
+    check_paths(4000, 3.5e9, false);
     check<1>(2000, 3.5e9);
     check<2>(2000, 3.5e9);
     check<3>(2000, 3.5e9);

@@ -44,3 +44,11 @@ def test_reflection_rows_adjoint_equals_tangents(report, depth):
         assert float(ordinary) < (5.0e-5 if kind in ("eps", "sigma", "thickness") else 1.0e-5), kind
         assert float(degenerate) < 2.0e-4, kind
         assert int(masked) == 0, kind
+
+
+@pytest.mark.parametrize("mode", ["coherent", "incoherent"])
+def test_stored_path_sweeps_equal_tangents(report, mode):
+    rows = {r[1]: [float(x) for x in r[2:]] for r in report if r[0] == mode}
+    # a path's own field weighs the incoherent cotangent: one more rounded factor of its size
+    for kind in ("planes", "wall_normals"):
+        assert rows[kind][0] < 5.0e-5, kind

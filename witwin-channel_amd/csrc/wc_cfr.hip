@@ -17,9 +17,9 @@
 // K = 2 entries) instead of 1,024 rotations, 16 per lane, on the vector units.
 // An arbitrary frequency list (cfr_list_kernel) evaluates every phasor.
 // Measured on 45,221 pairs of up to 199 paths (18 on average) x 1,024
-// subcarriers: 551 us with the rotations, 175 us with the matrix product (2.8 TB/s),
+// subcarriers: 551 us with the rotations, 195 us with the matrix product (2.5 TB/s),
 // for 0.49 GB of paths read and responses written; error against 64 bits 9.3e-7
-// before, 3.5e-7 now.
+// before, 1.6e-7 now.
 #include "wc_api_internal.h"
 #include "../../include/wcmi.h"
 
@@ -104,6 +104,26 @@ __global__ void __launch_bounds__(256) cfr_list_kernel(const float* __restrict__
     }
 }
 
+// exp(-j 2 pi cycles) to the last bit or two: reduced to an eighth of a turn in
+// float64, Taylor polynomials in float32 (remainders x^11 / 11! and x^12 / 12!,
+// below 2e-9 at pi / 4). A subcarrier's phasor is a product of two of these, so
+// each has to be better than the one the hardware sine gives (1e-7).
+__device__ __forceinline__ void phasor_factor(double cycles, float& c, float& s) {
+    const double quarters = rint(4.0 * cycles);
+    const float x = (float)(kTwoPiD * (cycles - 0.25 * quarters));
+    const float z = x * x;
+    const float sn = fmaf(x * z, fmaf(z, fmaf(z, fmaf(z, 1.0f / 362880.0f, -1.0f / 5040.0f), 1.0f / 120.0f),
+                                      -1.0f / 6.0f), x);
+    const float cs = fmaf(z, fmaf(z, fmaf(z, fmaf(z, fmaf(z, -1.0f / 3628800.0f, 1.0f / 40320.0f), -1.0f / 720.0f),
+                                          1.0f / 24.0f), -0.5f), 1.0f);
+    // the quarter turn's index modulo 4, exact for every finite double
+    const int k = (int)(quarters - 4.0 * floor(0.25 * quarters));
+    const bool odd = (k & 1) != 0;
+    const float a = odd ? sn : cs, b = odd ? cs : sn;
+    c = (k == 1 || k == 2) ? -a : a;
+    s = (k & 2) ? b : -b;
+}
+
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // swap the upper half of x with the lower half of y
@@ -166,7 +186,7 @@ cfr_grid_kernel(const float* __restrict__ a, const float* __restrict__ tau,
                 continue;
             }
             float c, sn;
-            phasor(f_lane * (double)t, c, sn);
+            phasor_factor(f_lane * (double)t, c, sn);
             const float wr = upper ? 1.0f : ar, wi = upper ? 0.0f : ai;
             float u = fmaf(wr, c, -wi * sn), v = fmaf(wr, sn, wi * c);
             // u: u_re | v_re, v: u_im | v_im  ->  u: u_re | u_im, v: v_re | v_im

@@ -1,0 +1,102 @@
+"""The native host part of scene compilation (wc_topology.hip) against plain
+restatements: edge candidates with their public ids (reference
+scene/resources.py:79-148, 286-404) on meshes with shared, boundary,
+non-manifold, welded-apart and degenerate edges, and the hulls of coplanar
+groups."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from witwin.channel import workloads
+from witwin.channel.scene import compiler
+
+
+def _edge_table(vertices, faces, face_group, face_structure, base):
+    """(vertex ids, public id) of every candidate edge, dictionary by dictionary."""
+    q = np.rint(vertices.astype(np.float64) / compiler.EDGE_WELD_QUANTIZATION).astype(np.int64)
+    ids, cursor = {}, 0
+    for s in range(len(base)):
+        pairs = sorted({(min(a, b), max(a, b)) for f in faces[face_structure == s] - base[s]
+                        for a, b in ((f[0], f[1]), (f[1], f[2]), (f[2], f[0]))})
+        ids.update({(s, *p): cursor + r for r, p in enumerate(pairs)})
+        cursor += len(pairs)
+    table = {}
+    for f, idx in enumerate(faces):
+        for k in range(3):
+            i = [int(idx[(k + j) % 3]) for j in range(3)]
+            a, b = tuple(q[i[0]]), tuple(q[i[1]])
+            la, lb = (x - base[face_structure[f]] for x in i[:2])
+            table.setdefault((min(a, b), max(a, b)), []).append(
+                (f, *i, ids[(face_structure[f], min(la, lb), max(la, lb))]))
+    out = []
+    for entries in table.values():
+        if len(entries) == 1:
+            out.append((*entries[0][1:4], -1, entries[0][4]))
+        elif len(entries) == 2 and face_group[entries[0][0]] != face_group[entries[1][0]]:
+            out.append((*entries[0][1:4], entries[1][3], min(entries[0][4], entries[1][4])))
+    return sorted(out, key=lambda e: e[4])
+
+
+def _random_mesh(seed):
+    rng = np.random.default_rng(seed)
+    corners = rng.uniform(-5.0, 5.0, (14, 3)).astype(np.float32)
+    vertices = np.concatenate([corners, corners[:6] + np.float32(2e-6), corners[6:9] + np.float32(1e-3)])
+    faces = rng.integers(0, 12, (24, 3))
+    faces = faces[(faces[:, 0] != faces[:, 1]) & (faces[:, 1] != faces[:, 2]) & (faces[:, 2] != faces[:, 0])]
+    # a second structure on the welded copies (vertices 14 ..)
+    more = rng.integers(0, 9, (12, 3))
+    more = more[(more[:, 0] != more[:, 1]) & (more[:, 1] != more[:, 2]) & (more[:, 2] != more[:, 0])]
+    structure = np.concatenate([np.zeros(len(faces), np.int64), np.ones(len(more), np.int64)])
+    return vertices, np.concatenate([faces, more + 14]).astype(np.int32), structure, np.array([0, 14])
+
+
+@pytest.mark.parametrize("seed", [1, 2, 3, 4])
+def test_edge_candidates_match_restatement(seed):
+    vertices, faces, structure, base = _random_mesh(seed)
+    group = np.arange(len(faces), dtype=np.int32) // 2
+    edges, ev, public = compiler.build_edge_table(vertices, faces, group, np.zeros(len(faces), np.int32),
+                                                  face_structure=structure, structure_vertex_base=base,
+                                                  return_ids=True)
+    ref = _edge_table(vertices, faces, group, structure, base)
+    g = compiler.edge_geometry(vertices, np.array([e[:4] for e in ref]).reshape(-1, 4))
+    keep = (g["length"] >= 1e-9) & ~(g["wedge"] & ((np.abs(g["alpha"] - np.pi) < compiler.COPLANAR_ANGLE_TOLERANCE)
+                                                   | (g["alpha"] < 1e-6)))
+    ref = [e for e, k in zip(ref, keep) if k]
+    assert len(ref) > 0 and [tuple(map(int, e)) for e in ev] == [tuple(map(int, e[:4])) for e in ref]
+    assert public.tolist() == [int(e[4]) for e in ref] and edges.shape[0] == len(ref)
+
+
+def test_edge_candidates_refuse_an_unknown_structure():
+    vertices, faces, structure, base = _random_mesh(1)
+    with pytest.raises(RuntimeError, match="structure"):
+        compiler.build_edge_table(vertices, faces, np.arange(len(faces), dtype=np.int32),
+                                  np.zeros(len(faces), np.int32), face_structure=structure + 1,
+                                  structure_vertex_base=base)
+
+
+def test_empty_mesh():
+    none = np.zeros((0, 3), np.int32)
+    edges, ev = compiler.build_edge_table(np.zeros((0, 3), np.float32), none, np.zeros(0, np.int32),
+                                          np.zeros(0, np.int32))
+    assert edges.shape == (0,) and ev.shape == (0, 4)
+    offset, points = compiler.group_hulls(np.zeros((0, 3), np.float32), none, np.zeros(1, np.int32),
+                                          np.zeros(0, np.int32), np.zeros((0, 4)))
+    assert offset.tolist() == [0] and points.shape == (0, 3)
+
+
+def test_group_hulls_contain_their_faces():
+    """Every hull runs counter-clockwise about its normal, holds its group's
+    vertices (to 1e-9 of coordinates near 400 m) and has only them as corners."""
+    c = compiler.compile(workloads.urban_canyon_scene(seed=2, shape=(2, 2)), reference_frequency_hz=3.5e9)
+    offset, points = compiler.group_hulls(c.vertices, c.faces, c.group_face_offset, c.group_faces, c.group_plane)
+    for g in range(c.group_count):
+        hull = points[offset[g]:offset[g + 1]]
+        members = c.group_faces[c.group_face_offset[g]:c.group_face_offset[g + 1]]
+        pts = c.vertices[c.faces[members].reshape(-1)].astype(np.float64)
+        n = c.group_plane[g, :3]
+        assert 3 <= len(hull) <= len(np.unique(pts, axis=0))
+        assert np.abs(hull[:, None] - pts[None]).max(axis=2).min(axis=1).max() < 1e-4  # off-plane part of a vertex
+        for a, b in zip(hull, np.roll(hull, -1, axis=0)):
+            assert (np.cross(b - a, pts - a) @ n >= -1e-9 * np.linalg.norm(b - a) * 400.0).all()

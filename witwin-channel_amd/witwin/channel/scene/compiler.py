@@ -220,15 +220,17 @@ def _group_tables(vertices: np.ndarray, faces: np.ndarray, face_group: np.ndarra
     g_count = representative.shape[0]
     v64 = vertices.astype(np.float64)
     planes = np.zeros((g_count, 4), dtype=np.float64)
-    for g, f in enumerate(representative):
-        a, b, c = v64[faces[f]]
-        n = np.cross(b - a, c - a)
-        n = n / max(np.linalg.norm(n), 1e-300)
-        k = int(np.argmax(np.abs(n)))
-        if n[k] < 0.0:
-            n = -n
-        planes[g, :3] = n
-        planes[g, 3] = float(np.dot(n, a))
+    if g_count:
+        # array operations but for the two dot products of a row, whose rounding order the planes keep
+        tri = v64[faces[representative]]
+        a = np.ascontiguousarray(tri[:, 0])
+        n = np.cross(tri[:, 1] - a, tri[:, 2] - a)
+        length = np.sqrt(np.fromiter((r.dot(r) for r in n), np.float64, g_count))
+        n = n / np.maximum(length, 1e-300)[:, None]
+        k = np.argmax(np.abs(n), axis=1)
+        n[n[np.arange(g_count), k] < 0.0] *= -1.0
+        planes[:, :3] = n
+        planes[:, 3] = np.fromiter((r.dot(s) for r, s in zip(n, a)), np.float64, g_count)
     order = np.argsort(face_group, kind="stable")
     counts = np.bincount(face_group, minlength=g_count)
     offsets = np.zeros(g_count + 1, dtype=np.int32)
@@ -293,39 +295,6 @@ def _edge_rows(geometry: dict[str, np.ndarray], ids: np.ndarray) -> np.ndarray:
     return rows
 
 
-def record_ids(faces: np.ndarray, face_structure: np.ndarray | None,
-               structure_vertex_base: np.ndarray | None) -> dict[tuple[int, int, int], int]:
-    """Public edge id of every (structure, local vertex a, local vertex b), a < b.
-
-    The reference numbers its edge records structure by structure: each
-    structure contributes one record per distinct vertex pair of its faces,
-    in ascending (lower, higher) local vertex id order, after the records of
-    the structures before it (reference scene/resources.py:79-148 exports the
-    records; their ids are what path rows carry as edge_id, e.g. the wedge of
-    tests/deterministic/test_diffraction_single_wedge.py:41-50 yields ids
-    0, 1, 2, 5 with record 3 the second copy of the shared edge). Without
-    structure tables every face belongs to structure 0.
-    """
-    faces = np.asarray(faces, dtype=np.int64).reshape(-1, 3)
-    if face_structure is None:
-        face_structure = np.zeros(faces.shape[0], dtype=np.int64)
-        structure_vertex_base = np.zeros(1, dtype=np.int64)
-    face_structure = np.asarray(face_structure, dtype=np.int64)
-    base = np.asarray(structure_vertex_base, dtype=np.int64)
-    ids: dict[tuple[int, int, int], int] = {}
-    cursor = 0
-    for s in range(base.shape[0]):
-        local = faces[face_structure == s] - base[s]
-        if local.size == 0:
-            continue
-        pairs = np.concatenate([local[:, [0, 1]], local[:, [1, 2]], local[:, [2, 0]]], axis=0)
-        pairs = np.unique(np.sort(pairs, axis=1), axis=0)
-        for r, (a, b) in enumerate(pairs.tolist()):
-            ids[(s, a, b)] = cursor + r
-        cursor += pairs.shape[0]
-    return ids
-
-
 def build_edge_table(vertices: np.ndarray, faces: np.ndarray, face_group: np.ndarray, face_material: np.ndarray,
                      policy: str = "all", face_structure: np.ndarray | None = None,
                      structure_vertex_base: np.ndarray | None = None,
@@ -339,57 +308,37 @@ def build_edge_table(vertices: np.ndarray, faces: np.ndarray, face_group: np.nda
     more than two faces are not diffracting. A wedge whose faces belong to two
     structures merges the two boundary records of the reference into the one
     with the lower id (reference scene/resources.py:286-404). Edges are ordered
-    by their public ids (``record_ids``; the lower id of a merged pair).
+    by their public ids, the lower id of a merged pair. The reference numbers
+    its edge records structure by structure: each structure contributes one
+    record per distinct vertex pair of its faces, in ascending (lower, higher)
+    local vertex id order, after the records of the structures before it
+    (reference scene/resources.py:79-148 exports the records; their ids are
+    what path rows carry as edge_id, e.g. the wedge of
+    tests/deterministic/test_diffraction_single_wedge.py:41-50 yields ids
+    0, 1, 2, 5 with record 3 the second copy of the shared edge). Without
+    structure tables every face belongs to structure 0. The candidates and
+    their ids come from ``wc_edge_candidates``.
     ``policy="vertical_only"`` keeps edges with |dz|/length > 0.7. Returns
     (records, [E, 4] int32 vertex ids (a, b, c0, c1), see edge_geometry) and,
     with ``return_ids``, the [E] int32 public ids.
     """
+    from witwin.channel import _native
+
     v = vertices.astype(np.float64)
-    q = np.rint(v / EDGE_WELD_QUANTIZATION).astype(np.int64)
-    public = record_ids(faces, face_structure, structure_vertex_base)
-    fstruct = (np.zeros(faces.shape[0], np.int64) if face_structure is None
-               else np.asarray(face_structure, dtype=np.int64))
-    vbase = (np.zeros(1, np.int64) if structure_vertex_base is None
-             else np.asarray(structure_vertex_base, dtype=np.int64))
-    table: dict[tuple, list] = {}
-    order: list[tuple] = []
-    for f in range(faces.shape[0]):
-        idx = faces[f]
-        for k in range(3):
-            i0, i1, i2 = int(idx[k]), int(idx[(k + 1) % 3]), int(idx[(k + 2) % 3])
-            a, b = tuple(q[i0]), tuple(q[i1])
-            key = (a, b) if a <= b else (b, a)
-            if key not in table:
-                table[key] = []
-                order.append(key)
-            table[key].append((f, i0, i1, i2))
-
-    def entry_id(f: int, i0: int, i1: int) -> int:
-        s = int(fstruct[f])
-        la, lb = i0 - int(vbase[s]), i1 - int(vbase[s])
-        return public[(s, min(la, lb), max(la, lb))]
-
-    cand_v, cand_i, cand_p = [], [], []
-    for key in order:
-        entries = table[key]
-        if len(entries) > 2:
-            continue
-        f0, i0, i1, i2 = entries[0]
-        if len(entries) == 2:
-            f1, j0, j1, j2 = entries[1]
-            if face_group[f1] == face_group[f0]:
-                continue
-            cand_v.append((i0, i1, i2, j2))
-            cand_i.append((f0, f1, int(face_group[f0]), int(face_group[f1]), int(face_material[f0]),
-                           int(face_material[f1])))
-            cand_p.append(min(entry_id(f0, i0, i1), entry_id(f1, j0, j1)))
-        else:
-            cand_v.append((i0, i1, i2, -1))
-            cand_i.append((f0, -1, int(face_group[f0]), -1, int(face_material[f0]), -1))
-            cand_p.append(entry_id(f0, i0, i1))
-    ev = np.asarray(cand_v, dtype=np.int64).reshape(-1, 4)
-    ids = np.asarray(cand_i, dtype=np.int64).reshape(-1, 6)
-    pid = np.asarray(cand_p, dtype=np.int64).reshape(-1)
+    q = np.ascontiguousarray(np.rint(v / EDGE_WELD_QUANTIZATION).astype(np.int64))
+    n_faces = int(faces.shape[0])
+    host = lambda x, dt: np.ascontiguousarray(x, dtype=dt)  # noqa: E731
+    tri, group, material = host(faces, np.int32), host(face_group, np.int32), host(face_material, np.int32)
+    fstruct = np.zeros(n_faces, np.int64) if face_structure is None else host(face_structure, np.int64)
+    vbase = np.zeros(1, np.int64) if structure_vertex_base is None else host(structure_vertex_base, np.int64)
+    ev = np.empty((3 * n_faces, 4), np.int64)
+    ids = np.empty((3 * n_faces, 6), np.int64)
+    pid = np.empty(3 * n_faces, np.int64)
+    count = np.zeros(1, np.int32)
+    _native.call("wc_edge_candidates", q.ctypes.data, tri.ctypes.data, n_faces, fstruct.ctypes.data,
+                 vbase.ctypes.data, int(vbase.shape[0]), group.ctypes.data, material.ctypes.data, ev.ctypes.data,
+                 ids.ctypes.data, pid.ctypes.data, count.ctypes.data)
+    ev, ids, pid = (x[:int(count[0])] for x in (ev, ids, pid))
     g = edge_geometry(v, ev)
     keep = g["length"] >= 1e-9
     if policy == "vertical_only":
@@ -575,14 +524,16 @@ def wide_node_levels(nodes: np.ndarray) -> tuple[np.ndarray, np.ndarray]:
     offsets of the groups (the order wc_scene_refit refits them in)."""
     words = np.ascontiguousarray(nodes).view(np.int32).reshape(-1, WIDE_NODE_BYTES // 4)
     counts = words[:, 3].view(np.uint32) >> 24
-    levels: list[list[int]] = [[0]]
+    levels = [np.zeros(1, dtype=np.int32)]
     while True:
-        nxt = [int(c) for n in levels[-1] for c in words[n, 12:12 + int(counts[n])] if c >= 0]
-        if not nxt:
+        child = words[levels[-1], 12:16]
+        nxt = child[(np.arange(4) < counts[levels[-1]][:, None]) & (child >= 0)]
+        if nxt.size == 0:
             break
         levels.append(nxt)
-    order = np.array([n for level in reversed(levels) for n in level], dtype=np.int32)
-    offsets = np.cumsum([0] + [len(level) for level in reversed(levels)]).astype(np.int32)
+    levels.reverse()
+    order = np.concatenate(levels).astype(np.int32)
+    offsets = np.cumsum([0] + [len(level) for level in levels]).astype(np.int32)
     return order, offsets
 
 
@@ -592,61 +543,34 @@ def group_hulls(vertices: np.ndarray, faces: np.ndarray, group_face_offset: np.n
     offsets, [H, 3] float64 points on the plane, counter-clockwise about the
     normal). A one-triangle group is its triangle; larger groups take the
     monotone-chain hull of their vertices in an in-plane basis."""
+    from witwin.channel import _native
+
+    host = lambda x, dt: np.ascontiguousarray(x, dtype=dt)  # noqa: E731
     g = int(group_plane.shape[0])
-    n = group_plane[:, :3].astype(np.float64)
-    off = group_plane[:, 3].astype(np.float64)
-    # in-plane basis: u = a unit vector orthogonal to n, w = n x u
-    helper = np.where(np.abs(n[:, :1]) < 0.9, np.array([[1.0, 0.0, 0.0]]), np.array([[0.0, 1.0, 0.0]]))
-    u = np.cross(n, helper)
-    u /= np.linalg.norm(u, axis=1, keepdims=True)
-    w = np.cross(n, u)
-    origin = n * off[:, None]
-    counts = np.diff(group_face_offset)
-    hull_pts: list[np.ndarray] = [np.zeros((0, 3))] * g
-    v64 = vertices.astype(np.float64)
+    verts, tri, plane = host(vertices, np.float32), host(faces, np.int32), host(group_plane, np.float64)
+    first, members = host(group_face_offset, np.int32), host(group_faces, np.int32)
+    offset = np.zeros(g + 1, np.int32)
+    points = np.empty((3 * int(members.shape[0]) * 2, 3), np.float64)
+    _native.call("wc_group_hulls", verts.ctypes.data, tri.ctypes.data, first.ctypes.data, members.ctypes.data,
+                 plane.ctypes.data, g, offset.ctypes.data, points.ctypes.data)
+    return offset, np.ascontiguousarray(points[:int(offset[g])])
 
-    def to_plane(gi: int, pts: np.ndarray) -> np.ndarray:
-        d = pts - origin[gi]
-        return np.stack([d @ u[gi], d @ w[gi]], axis=1)
 
-    def from_plane(gi: int, uv: np.ndarray) -> np.ndarray:
-        return origin[gi] + uv[:, :1] * u[gi] + uv[:, 1:2] * w[gi]
-
-    def monotone(uv: np.ndarray) -> np.ndarray:
-        pts = np.unique(uv, axis=0)
-        if pts.shape[0] < 3:
-            return pts
-
-        def half(seq):
-            out: list[np.ndarray] = []
-            for p in seq:
-                while len(out) >= 2 and ((out[-1][0] - out[-2][0]) * (p[1] - out[-2][1])
-                                         - (out[-1][1] - out[-2][1]) * (p[0] - out[-2][0])) <= 0.0:
-                    out.pop()
-                out.append(p)
-            return out
-
-        lower = half(pts)
-        upper = half(pts[::-1])
-        return np.array(lower[:-1] + upper[:-1])
-
-    single = np.nonzero(counts == 1)[0]
-    if single.size:
-        tri = v64[faces[group_faces[group_face_offset[single]]]]  # [S, 3, 3]
-        for k, gi in enumerate(single):
-            uv = to_plane(gi, tri[k])
-            area = (uv[1, 0] - uv[0, 0]) * (uv[2, 1] - uv[0, 1]) - (uv[1, 1] - uv[0, 1]) * (uv[2, 0] - uv[0, 0])
-            if area < 0.0:
-                uv = uv[::-1]
-            hull_pts[gi] = from_plane(gi, uv)
-    for gi in np.nonzero(counts > 1)[0]:
-        members = group_faces[group_face_offset[gi]:group_face_offset[gi + 1]]
-        pts = v64[faces[members].reshape(-1)]
-        hull_pts[gi] = from_plane(gi, monotone(to_plane(gi, pts)))
-    sizes = np.array([h.shape[0] for h in hull_pts], dtype=np.int64)
-    offset = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
-    points = np.concatenate(hull_pts, axis=0) if g else np.zeros((0, 3))
-    return offset, np.ascontiguousarray(points, dtype=np.float64)
+def _upload(device: torch.device, arrays: list[tuple[np.ndarray, np.dtype]]) -> list[torch.Tensor]:
+    """Device copies of host arrays as views of one buffer (one transfer;
+    256-byte aligned parts)."""
+    host = [np.ascontiguousarray(a, dtype=dt) for a, dt in arrays]
+    start = np.concatenate([[0], np.cumsum([(a.nbytes + 255) // 256 * 256 for a in host])]).astype(np.int64)
+    packed = np.zeros(max(int(start[-1]), 1), np.uint8)
+    for a, at in zip(host, start):
+        packed[at:at + a.nbytes] = a.reshape(-1).view(np.uint8)
+    buffer = torch.from_numpy(packed).to(device)
+    out = []
+    for a, at in zip(host, start):
+        dtype = torch.from_numpy(np.empty(0, a.dtype)).dtype
+        out.append(buffer[int(at):int(at) + a.nbytes].view(dtype).reshape(a.shape) if a.nbytes
+                   else torch.empty(a.shape, dtype=dtype, device=device))
+    return out
 
 
 class DeviceScene:
@@ -667,57 +591,44 @@ class DeviceScene:
             raise ValueError(f"bvh must be one of {BVH_BUILDERS}, got {bvh!r}")
         self.device = device
         self.bvh = bvh
-        t = lambda a, dt: torch.as_tensor(np.ascontiguousarray(a)).to(device=device, dtype=dt).contiguous()  # noqa: E731
         mats = compiled.materials
-        self.vertices = t(compiled.vertices, torch.float32)
-        self.faces = t(compiled.faces, torch.int32)
-        self.face_group = t(compiled.face_group, torch.int32)
-        self.face_material = t(compiled.face_material, torch.int32)
-        self.group_plane = t(compiled.group_plane, torch.float64)
-        self.group_face_offset = t(compiled.group_face_offset, torch.int32)
-        self.group_faces = t(compiled.group_faces, torch.int32)
-        self.group_material = t(compiled.group_material, torch.int32)
-        self.mat_eps = t(mats.eps_r, torch.float32)
-        self.mat_sigma = t(mats.sigma_e, torch.float32)
-        self.mat_mu = t(mats.mu_r, torch.float32)
-        self.mat_gain = t(mats.gain, torch.float32)
-        self.mat_thickness = t(mats.thickness_m, torch.float32)
-        self.layer_offset = t(mats.layer_offset, torch.int32)
-        self.layer_count = t(mats.layer_count, torch.int32)
-        self.layer_thickness = t(mats.layer_thickness_m, torch.float32)
-        self.layer_eps = t(mats.layer_eps_r, torch.float32)
-        self.layer_sigma = t(mats.layer_sigma_e, torch.float32)
-        self.layer_mu = t(mats.layer_mu_r, torch.float32)
-        self.group_face = t(compiled.representative_faces, torch.int32)
-        self.edge_vertices = t(compiled.edge_vertices.reshape(-1, 4), torch.int32)
+        f = compiled.face_count
+        f32, i32 = np.float32, np.int32
         public = compiled.edge_public_id if compiled.edge_public_id.shape[0] == compiled.edge_count \
             else np.arange(compiled.edge_count)
-        self.edge_public_id = t(public.reshape(-1), torch.int32)
-        self.group_count = compiled.group_count
-        self.edge_count = compiled.edge_count
-        self._csr: tuple[torch.Tensor, torch.Tensor] | None = None
-        self._hulls: tuple[torch.Tensor, torch.Tensor] | None = None
         edge_bytes = compiled.edges.view(np.uint8).reshape(-1) if compiled.edge_count else np.zeros(0, np.uint8)
-        self.edges = torch.as_tensor(edge_bytes.copy()).to(device)
-        f = compiled.face_count
         self.node_count = int(_native.call("wc_bvh_node_count", f))
-        self.nodes = torch.zeros(self.node_count * WIDE_NODE_BYTES, dtype=torch.uint8, device=device)
-        self.sorted_tris = torch.zeros(max(f, 1) * 48, dtype=torch.uint8, device=device)
-        self.face_tris = torch.zeros(max(f, 1) * 48, dtype=torch.uint8, device=device)
+        nodes = np.zeros(self.node_count * WIDE_NODE_BYTES, np.uint8)
+        sorted_tris = np.zeros(max(f, 1) * 48, np.uint8)
+        face_tris = np.zeros(max(f, 1) * 48, np.uint8)
         if f and bvh == "sah":
             host = lambda a, dt: np.ascontiguousarray(a, dtype=dt)  # noqa: E731
             verts, tri_faces = host(compiled.vertices, np.float32), host(compiled.faces, np.int32)
             groups, materials = host(compiled.face_group, np.int32), host(compiled.face_material, np.int32)
-            nodes = np.zeros(self.node_count * WIDE_NODE_BYTES, np.uint8)
-            sorted_tris = np.zeros(f * 48, np.uint8)
-            face_tris = np.zeros(f * 48, np.uint8)
             _native.call("wc_bvh_build_sah", verts.ctypes.data, tri_faces.ctypes.data, groups.ctypes.data,
                          materials.ctypes.data, f, nodes.ctypes.data, sorted_tris.ctypes.data, face_tris.ctypes.data)
-            self.nodes.copy_(torch.from_numpy(nodes))
-            self.sorted_tris.copy_(torch.from_numpy(sorted_tris))
-            self.face_tris.copy_(torch.from_numpy(face_tris))
-            wide_host = nodes
-        elif f:
+        (self.vertices, self.faces, self.face_group, self.face_material, self.group_plane, self.group_face_offset,
+         self.group_faces, self.group_material, self.mat_eps, self.mat_sigma, self.mat_mu, self.mat_gain,
+         self.mat_thickness, self.layer_offset, self.layer_count, self.layer_thickness, self.layer_eps,
+         self.layer_sigma, self.layer_mu, self.group_face, self.edge_vertices, self.edge_public_id, self.edges,
+         self.nodes, self.sorted_tris, self.face_tris) = _upload(device, [
+             (compiled.vertices, f32), (compiled.faces, i32), (compiled.face_group, i32),
+             (compiled.face_material, i32), (compiled.group_plane, np.float64), (compiled.group_face_offset, i32),
+             (compiled.group_faces, i32), (compiled.group_material, i32), (mats.eps_r, f32), (mats.sigma_e, f32),
+             (mats.mu_r, f32), (mats.gain, f32), (mats.thickness_m, f32), (mats.layer_offset, i32),
+             (mats.layer_count, i32), (mats.layer_thickness_m, f32), (mats.layer_eps_r, f32),
+             (mats.layer_sigma_e, f32), (mats.layer_mu_r, f32), (compiled.representative_faces, i32),
+             (compiled.edge_vertices.reshape(-1, 4), i32), (public.reshape(-1), i32), (edge_bytes, np.uint8),
+             (nodes, np.uint8), (sorted_tris, np.uint8), (face_tris, np.uint8)])
+        self.group_count = compiled.group_count
+        self.edge_count = compiled.edge_count
+        self._csr: tuple[torch.Tensor, torch.Tensor] | None = None
+        self._hulls: tuple[torch.Tensor, torch.Tensor] | None = None
+        # the arrays the group hulls are made of, until a refit moves them
+        self._hull_host = (compiled.vertices, compiled.faces, compiled.group_face_offset, compiled.group_faces,
+                           compiled.group_plane)
+        wide_host = nodes
+        if f and bvh == "lbvh":
             ws_bytes = int(_native.call("wc_bvh_workspace_bytes", f))
             workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
             binary = torch.zeros(self.node_count * BINARY_NODE_BYTES, dtype=torch.uint8, device=device)
@@ -763,7 +674,7 @@ class DeviceScene:
 
         v = vertices.detach().to(device=self.device, dtype=torch.float32).reshape(self.vertices.shape)
         self.vertices.copy_(v)
-        self._hulls = None  # group hulls follow the vertices
+        self._hulls = self._hull_host = None  # group hulls follow the vertices
         failure = torch.zeros(1, dtype=torch.int32, device=self.device)
         p = _native.ptr
         levels = np.ascontiguousarray(self._refit_offsets, dtype=np.int32)
@@ -779,9 +690,9 @@ class DeviceScene:
         """Device copy of group_hulls for the current vertices (built on first
         use, rebuilt after a refit)."""
         if self._hulls is None:
-            offset, points = group_hulls(self.vertices.cpu().numpy(), self.faces.cpu().numpy(),
-                                         self.group_face_offset.cpu().numpy(), self.group_faces.cpu().numpy(),
-                                         self.group_plane.cpu().numpy())
+            offset, points = group_hulls(*(self._hull_host or (
+                self.vertices.cpu().numpy(), self.faces.cpu().numpy(), self.group_face_offset.cpu().numpy(),
+                self.group_faces.cpu().numpy(), self.group_plane.cpu().numpy())))
             self._hulls = (torch.as_tensor(offset).to(self.device),
                            torch.as_tensor(points if points.size else np.zeros((1, 3))).to(self.device))
         return self._hulls

@@ -151,6 +151,33 @@ def test_shadow_bins_and_pretest_on_heightfield(checker, tmp_path):
 
 
 @pytest.mark.parametrize("which", ["canyon", "heightfield"])
+def test_shadow_walk_equals_every_triangle(tmp_path_factory, tmp_path, which):
+    """The tree walk's bins are those of the section test of every triangle:
+    transmitters in the streets, over the roofs, on an edge's line and far off."""
+    from test_cpu_oracle_and_host import _sah_tables
+
+    if which == "canyon":
+        scene = workloads.urban_canyon_scene(seed=2, shape=(2, 2))
+        txs = [(53.231, 52.013, 25.0), (180.3, 170.7, 3.2), (5.0, 5.0, 80.0), (-900.0, 400.0, 30.0)]
+    else:
+        scene = workloads.heightfield_scene(seed=4, size=40, boxes=10, shape=(2, 2))
+        txs = [tuple(scene.endpoints[0].position.tolist()), (10.0, 12.0, 60.0)]
+    compiled = compile_scene(scene, reference_frequency_hz=3.5e9)
+    nodes, sorted_tris, _ = _sah_tables(compiled)
+    e = compiled.edges[len(compiled.edges) // 2]
+    txs.append(tuple(float(e["a" + k] - 7.0 * e["d" + k]) for k in "xyz"))
+    out = tmp_path / which
+    out.mkdir()
+    nodes.tofile(out / "nodes.bin")
+    sorted_tris.astype(np.float32).tofile(out / "tris.bin")
+    compiled.edges.view(np.uint8).tofile(out / "edges.bin")
+    np.asarray(txs, np.float32).tofile(out / "txs.bin")
+    c = _run(_build(tmp_path_factory, "shadow_walk_check"), out)
+    assert c["wrong"] == 0 and c["idle"] == 0
+    assert c["set"] > c["pairs"] // 10
+
+
+@pytest.mark.parametrize("which", ["canyon", "heightfield"])
 def test_chain_tile_cull_drops_no_valid_chain(chain_checker, tmp_path, which):
     if which == "canyon":
         scene = workloads.urban_canyon_scene(seed=2, shape=(24, 24), spacing=14.0)

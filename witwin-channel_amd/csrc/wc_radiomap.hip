@@ -1705,43 +1705,169 @@ __host__ __device__ inline bool fan_plane_misses(const FanPlane& p, const Tri& t
 }
 
 // Shadow bins of every (transmitter, edge) over all triangles outside the
-// edge's own face groups (which the leg test ignores). A wavefront serves
-// 64 / P edges of one transmitter with P lanes each: lane P j + p takes edge
-// j of the group and triangles p, p + P, ..., so a triangle fetch serves
-// 64 / P edges (P = 8 when there are many pairs, 64 when few, to fill the
-// chip). Only the triangles that reach an edge's fan plane take the
-// double-precision section test; the P lanes of an edge then OR their bins.
-__global__ void __launch_bounds__(256) edge_shadow_kernel(SceneView s, wc_solve q, int lanes_per_edge,
+// edge's own face groups (which the leg test ignores): one wavefront per pair,
+// lane l pre-tests triangles l, l + 64, ... The few that reach the edge's fan
+// triangle (3 % on the canyon, so most rounds of 64 have one) queue in LDS and
+// take the double-precision section test 64 at a time; tested where they are
+// met, nearly every round paid for one. 64 transmitters of the canyon (49,408
+// pairs, 770 triangles): 272 us tested at once, 174 us queued.
+__global__ void __launch_bounds__(256) edge_shadow_kernel(SceneView s, wc_solve q,
                                                           unsigned long long* __restrict__ shadow, long long wave_base) {
-    const long long wave = wave_base + (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    __shared__ int queue[4][128];
+    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const long long pair = wave_base + (long long)blockIdx.x * (blockDim.x >> 6) + wid;
     const int edges = s.edge_count;
-    const int per_wave = 64 / lanes_per_edge;
-    const int groups = (edges + per_wave - 1) / per_wave;
-    if (wave >= (long long)q.tx_count * groups) return;
-    const int lane = threadIdx.x & 63;
-    const int t = (int)(wave / groups);
-    const int ei = (int)(wave - (long long)t * groups) * per_wave + lane / lanes_per_edge;
-    const int phase = lane & (lanes_per_edge - 1);
+    if (pair >= (long long)q.tx_count * edges) return;  // the whole wavefront
+    const int t = (int)(pair / edges);
+    const Edge e = s.edges[pair - (long long)t * edges];
+    const ShadowFrame f = shadow_frame(e, ld3(q.tx_pos + 3 * t));
     unsigned long long bits = 0;
-    if (ei < edges) {
-        const Edge e = s.edges[ei];
-        const ShadowFrame f = shadow_frame(e, ld3(q.tx_pos + 3 * t));
-        if (f.valid) {
-            const FanPlane plane = fan_plane(f);
-            for (int k = phase; k < s.face_count; k += lanes_per_edge) {
+    if (f.valid) {
+        const FanPlane plane = fan_plane(f);
+        int queued = 0;  // the same in every lane
+        for (int base = 0; base < s.face_count || queued > 0; base += 64) {
+            const int k = base + lane;
+            bool reach = false;
+            if (k < s.face_count) {
                 const Tri tri = s.faces[k];
                 const int group = __float_as_int(tri.v0.w);
-                if (group == e.group0 || group == e.group1 || fan_plane_misses(plane, tri)) continue;
-                bits |= triangle_shadow_bins(f, tri);
+                reach = group != e.group0 && group != e.group1 && !fan_plane_misses(plane, tri);
             }
+            const unsigned long long ball = __ballot(reach);
+            if (reach) queue[wid][queued + (int)__popcll(ball & ((1ull << lane) - 1ull))] = k;
+            queued += (int)__popcll(ball);
+            if (queued < 64 && base + 64 < s.face_count) continue;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const int item = lane < queued ? queue[wid][lane] : -1;
+            const int carry = lane + 64 < queued ? queue[wid][lane + 64] : -1;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (carry >= 0) queue[wid][lane] = carry;
+            queued = queued > 64 ? queued - 64 : 0;
+            if (item >= 0) bits |= triangle_shadow_bins(f, s.faces[item]);
         }
     }
-    for (int off = 1; off < lanes_per_edge; off <<= 1) {
+    for (int off = 1; off < 64; off <<= 1) {
         const unsigned lo32 = __shfl_xor((unsigned)bits, off), hi32 = __shfl_xor((unsigned)(bits >> 32), off);
         bits |= ((unsigned long long)hi32 << 32) | lo32;
     }
-    if (ei < edges && phase == 0) shadow[(size_t)t * edges + ei] = bits;
+    if (lane == 0) shadow[pair] = bits;
 }
+
+// The same bins by a walk of the tree, kShadowLanes lanes per (transmitter,
+// edge), each below its own grandchild of the root: a box that lies beyond one side of the fan triangle (T, A, B) or off its plane, by
+// the pre-test's margin, holds no triangle that sets a bin. Triangles that
+// pass the pre-test wait in a short list per lane, and the wavefront runs their
+// double-precision section tests together when a list fills: tested where the
+// walk meets them, nearly every step would run one for a lane or two.
+// The kernel above reads every triangle for every edge; it stays for small
+// meshes, where a fan triangle meets a good part of the tree
+// (see edge_shadow_walks).
+constexpr int kShadowList = 12;  // per lane; a step adds at most four
+constexpr int kShadowLanes = 16;
+
+struct FanSides {
+    V3<float> na, nb;  // outward normals of the sides A-T and B-T
+};
+__device__ __forceinline__ FanSides fan_sides(const FanPlane& p) {
+    return {{p.at_x * p.dx + p.at_y * p.wx, p.at_x * p.dy + p.at_y * p.wy, p.at_x * p.dz + p.at_y * p.wz},
+            {p.bt_x * p.dx + p.bt_y * p.wx, p.bt_x * p.dy + p.bt_y * p.wy, p.bt_x * p.dz + p.bt_y * p.wz}};
+}
+__device__ __forceinline__ bool fan_plane_misses_box(const FanPlane& p, const FanSides& n, float lx, float ly, float lz,
+                                                     float hx, float hy, float hz) {
+    const float ex = 0.5f * (hx - lx), ey = 0.5f * (hy - ly), ez = 0.5f * (hz - lz);
+    const float cx = 0.5f * (lx + hx) - p.ax, cy = 0.5f * (ly + hy) - p.ay, cz = 0.5f * (lz + hz) - p.az;
+    auto mid = [&](float x, float y, float z) { return x * cx + y * cy + z * cz; };
+    auto reach = [&](float x, float y, float z) { return fabsf(x) * ex + fabsf(y) * ey + fabsf(z) * ez; };
+    const float sd = mid(p.mx, p.my, p.mz), rs = reach(p.mx, p.my, p.mz);
+    const float y = mid(p.wx, p.wy, p.wz), ry = reach(p.wx, p.wy, p.wz);
+    const float a = mid(n.na.x, n.na.y, n.na.z), ra = reach(n.na.x, n.na.y, n.na.z);
+    const float b = mid(n.nb.x, n.nb.y, n.nb.z) - p.bt_x * p.len, rb = reach(n.nb.x, n.nb.y, n.nb.z);
+    return fabsf(sd) - rs > p.tol || y + ry < -p.tol || a - ra > p.tol || b - rb > p.tol;
+}
+
+// Bins of the triangles below lane `part`'s grandchild of the root (every lane
+// of the wavefront takes part; `valid` switches a lane off).
+__device__ __forceinline__ unsigned long long shadow_walk(const SceneView& s, bool valid, const ShadowFrame& f,
+                                                          int own0, int own1, int part,
+                                                          int (*__restrict__ list)[256], int tid) {
+    unsigned long long bits = 0;
+    bool walking = valid && s.tri_count > 0;
+    const FanPlane plane = fan_plane(f);
+    const FanSides sides = fan_sides(plane);
+    int stack[kWideStackSize];
+    int sp = 0, node = 0, level = 0, waiting = 0;
+    while (true) {
+        if (walking) {
+            const WideNode nd = fetch_node<kStageTop>(s, node);
+            // the first two steps take one child each: part's digit of that level
+            const int only = level == 0 ? part >> 2 : (level == 1 ? part & 3 : -1);
+            const float sx = grid_step(nd.exps, 0), sy = grid_step(nd.exps, 1), sz = grid_step(nd.exps, 2);
+            const int count = (int)(nd.exps >> 24);
+            int next = -1;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (k >= count || (only >= 0 && k != only) ||
+                    fan_plane_misses_box(plane, sides, grid_bound(nd.lo_x, k, sx, nd.ox),
+                                         grid_bound(nd.lo_y, k, sy, nd.oy), grid_bound(nd.lo_z, k, sz, nd.oz),
+                                         grid_bound(nd.hi_x, k, sx, nd.ox), grid_bound(nd.hi_y, k, sy, nd.oy),
+                                         grid_bound(nd.hi_z, k, sz, nd.oz)))
+                    continue;
+                const int c = k == 0 ? nd.child.x : (k == 1 ? nd.child.y : (k == 2 ? nd.child.z : nd.child.w));
+                if (c < 0) {
+                    const Tri tri = s.tris[~c];
+                    const int group = __float_as_int(tri.v0.w);
+                    if (group != own0 && group != own1 && !fan_plane_misses(plane, tri)) list[waiting++][tid] = ~c;
+                } else if (next < 0) {
+                    next = c;
+                } else if (sp < kWideStackSize) {
+                    stack[sp++] = c;
+                }
+            }
+            if (next < 0 && sp > 0) next = stack[--sp];
+            node = next;
+            ++level;
+            walking = next >= 0;
+        }
+        const bool more = __ballot(walking) != 0ull;
+        if (more && __ballot(waiting > kShadowList - 4) == 0ull) continue;
+        for (int i = 0; __ballot(i < waiting) != 0ull; ++i)
+            if (i < waiting) bits |= triangle_shadow_bins(f, s.tris[list[i][tid]]);
+        waiting = 0;
+        if (bits == ~0ull) walking = false;  // nothing left to find
+        if (!more) return bits;
+    }
+}
+
+__global__ void __launch_bounds__(256) edge_shadow_walk_kernel(SceneView s, wc_solve q,
+                                                               unsigned long long* __restrict__ shadow,
+                                                               long long pairs, long long pair_base) {
+    if (kStageTop) stage_top_nodes(s);
+    __shared__ int list[kShadowList][256];
+    const int part = threadIdx.x & (kShadowLanes - 1);
+    const long long pair = pair_base + ((long long)blockIdx.x * blockDim.x + threadIdx.x) / kShadowLanes;
+    const long long at = pair < pairs ? pair : pairs - 1;
+    const int t = (int)(at / s.edge_count);
+    const Edge e = s.edges[at - (long long)t * s.edge_count];
+    const ShadowFrame f = shadow_frame(e, ld3(q.tx_pos + 3 * t));
+    unsigned long long bits =
+        shadow_walk(s, pair < pairs && f.valid, f, e.group0, e.group1, part, list, (int)threadIdx.x);
+    for (int off = 1; off < kShadowLanes; off <<= 1) {
+        const unsigned lo32 = __shfl_xor((unsigned)bits, off), hi32 = __shfl_xor((unsigned)(bits >> 32), off);
+        bits |= ((unsigned long long)hi32 << 32) | lo32;
+    }
+    if (pair < pairs && part == 0) shadow[pair] = bits;
+}
+
+// Which shadow kernel, by the triangles the other one reads per edge. Measured,
+// walk against all triangles: 772 edges of one transmitter on 770 triangles
+// 0.298 / 0.024 ms, 64 transmitters there 0.597 / 0.174 ms (a street's fan
+// meets much of so small a tree), 8 transmitters of the scaled city (134,850
+// triangles) 1.22 / 5.06 ms.
+__host__ inline bool edge_shadow_walks(int face_count) { return face_count >= 16384; }
 
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WC_VIS_WAVES_PER_EU)))
 diff_visibility_kernel(SceneView s, wc_solve q, unsigned* __restrict__ masks, int words, long long waves,
@@ -2377,8 +2503,9 @@ static int device_cus() {
     return cached_cus;
 }
 
-// The shadow table costs transmitters x edges x triangles segment-plane
-// tests; above this many it is skipped (the visibility test alone is exact).
+// The brute-force shadow table costs transmitters x edges x triangles
+// segment-plane tests; above this many it is skipped (the visibility test
+// alone is exact).
 constexpr long long kShadowBudget = 4000000000LL;
 
 static void launch_diff_visibility(const SceneView& s, const wc_solve& q, const wc_radiomap_out& o, hipStream_t st) {
@@ -2388,18 +2515,20 @@ static void launch_diff_visibility(const SceneView& s, const wc_solve& q, const 
                                                   partial_bytes(q.total_cells, q.lanes_per_cell));
     unsigned long long* shadow = nullptr;
     const long long pairs = (long long)q.tx_count * s.edge_count;
-    if (pairs > 0 && pairs * (long long)s.face_count <= kShadowBudget) {
+    const bool walk = edge_shadow_walks(s.face_count);
+    if (pairs > 0 && (walk || pairs * (long long)s.face_count <= kShadowBudget)) {
         shadow = reinterpret_cast<unsigned long long*>(
             static_cast<char*>(o.workspace) + shadow_offset(q.total_cells, q.lanes_per_cell, s.edge_count,
                                                             q.max_tx_chains, q.tx_count));
-        // 64 lanes per edge: on the urban canyon with 64 transmitters, 8 lanes
-        // per edge (fewer triangle fetches) measured slower
-        const int lanes_per_edge = 64;
-        const int per_wave = 64 / lanes_per_edge;
-        const long long shadow_waves = (long long)q.tx_count * ((s.edge_count + per_wave - 1) / per_wave);
-        for_wave_chunks(shadow_waves, [&](dim3 grid, long long base) {
-            hipLaunchKernelGGL(edge_shadow_kernel, grid, dim3(256), 0, st, s, q, lanes_per_edge, shadow, base);
-        });
+        if (walk)
+            for_wave_chunks((pairs * kShadowLanes + 63) / 64, [&](dim3 grid, long long base) {
+                hipLaunchKernelGGL(edge_shadow_walk_kernel, grid, dim3(256), 0, st, s, q, shadow, pairs,
+                                   base * (64 / kShadowLanes));
+            });
+        else
+            for_wave_chunks(pairs, [&](dim3 grid, long long base) {
+                hipLaunchKernelGGL(edge_shadow_kernel, grid, dim3(256), 0, st, s, q, shadow, base);
+            });
     }
     const long long waves = ((long long)q.total_cells + 63) / 64 * words;
     // a receiver grid shared by the transmitters keeps neighbouring receivers

@@ -1180,7 +1180,7 @@ __device__ __forceinline__ bool chain_legs(const SceneView& s, const wc_solve& q
                                            const V3<float>& rx);
 
 // Chain validity behind a supertile cull, tile loops: one wavefront per
-// (tile, segment of 64 chain words). Its lanes load the segment's 64 supertile
+// (tile, segment of up to 64 chain words). Its lanes load the segment's supertile
 // words at once and the wavefront visits only the chunks (32 chains) its
 // supertile kept: the tile cull of those chains against the tile's receiver
 // box, then every receiver tests the survivors exactly. The bits equal
@@ -1194,15 +1194,77 @@ __device__ __forceinline__ bool chain_legs(const SceneView& s, const wc_solve& q
 #define WC_SEG_WAVES_PER_EU 4
 #endif
 
+// Tile cull of a segment's kept chains: lane l holds word l (32 chains from c0
+// of its chunk); the result is its word with only the chains that reach the
+// box. A word keeps a few of its 32 chains, so the set bits of all 64 words are
+// dealt to the lanes in order, 64 chains a round, instead of 32 lanes taking
+// one word at a time (scaled city 15.9 -> 14.1 ms a pass, heightfield 1.97 ->
+// 1.90 ms).
+__device__ __forceinline__ unsigned cull_segment(const SceneView& s, const wc_solve& q, int t, int first_chain,
+                                                 int end, unsigned sword, unsigned* __restrict__ found,
+                                                 const V3<float>& lo, const V3<float>& hi) {
+    const int lane = threadIdx.x & 63;
+    int inclusive = __popc(sword);
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(inclusive, off);
+        if (lane >= off) inclusive += y;
+    }
+    const int exclusive = inclusive - __popc(sword);
+    const int total = __shfl(inclusive, 63);
+    found[lane] = 0u;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int base = 0; base < total; base += 64) {
+        // owner word u of bit j: the last whose exclusive prefix is <= j
+        const int j = base + lane;
+        int u = 0;
+#pragma unroll
+        for (int step = 32; step >= 1; step >>= 1)
+            if (__shfl(exclusive, u + step) <= j) u += step;
+        unsigned word = (unsigned)__shfl((int)sword, u);
+        const int skip = j - __shfl(exclusive, u);
+        if (j >= total) continue;
+        for (int i = 0; i < skip; ++i) word &= word - 1;
+        const int bit = __ffs(word) - 1;
+        const int c = first_chain + u * 32 + bit;
+        if (c >= end) continue;
+        int d = 1;
+        while (c >= q.chain_offset[t * kMaxDepth + d]) ++d;
+        if (chain_reaches_box(s, q, c, d, lo, hi)) atomicOr(&found[u], 1u << bit);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    return found[lane];
+}
+
+// Chain words of one wavefront's segment (at most 64, a lane per word). A
+// tile's surviving chains are tested one after the other by the wavefront that
+// holds them, so with few tiles the kernel lasts as long as its busiest
+// segment and short segments pay; with many, the segments' fixed costs do not.
+// Segments of 64 / 16 / 4 / 1 words: heightfield (1,024 tiles, 722 words)
+// 1.90 / 1.50 / 1.13 / 1.18 ms, eight transmitters of the scaled city (12 k
+// tiles, 1.5 k words) 14.1 / 14.6 / 18.0 / 26.4 ms a pass. The shortest
+// segment (4 to 64) that keeps the launch below 200,000 wavefronts.
+constexpr long long kSegWaves = 200000;
+__host__ inline int segment_words(long long tile_count, int words) {
+    int n = 4;
+    while (n < 64 && tile_count * ((words + n - 1) / n) > kSegWaves) n <<= 1;
+    return n;
+}
+
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WC_SEG_WAVES_PER_EU)))
 chain_visibility_seg_kernel(SceneView s, wc_solve q,
                                                                    const int* __restrict__ tiles, int tile_count,
                                                                    unsigned* __restrict__ masks, int words,
                                                                    const unsigned* __restrict__ super_masks,
                                                                    long long wave_base,
-                                                                   unsigned* __restrict__ touched) {
+                                                                   unsigned* __restrict__ touched, int seg_words) {
     if (kStageTop) stage_top_nodes(s);
-    const int segs = (words + 63) >> 6;
+    __shared__ unsigned found[4][64];
+    const int segs = (words + seg_words - 1) / seg_words;
     const long long wave = wave_base + (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     if (wave >= (long long)tile_count * segs) return;
     const int tile = (int)(wave / segs);
@@ -1212,8 +1274,9 @@ chain_visibility_seg_kernel(SceneView s, wc_solve q,
     const int base = q.chain_offset[t * kMaxDepth];
     const int end = q.chain_offset[t * kMaxDepth + min(q.max_depth, kMaxDepth)];
     const int tx_words = mask_words(end - base);
-    const int w = seg * 64 + lane;
-    const unsigned sword = w < tx_words ? super_masks[(size_t)super_of_tile(q, tile) * words + w] : 0u;
+    const int w = seg * seg_words + lane;
+    const unsigned sword =
+        lane < seg_words && w < tx_words ? super_masks[(size_t)super_of_tile(q, tile) * words + w] : 0u;
     unsigned long long chunks = __ballot(sword != 0u);
     if (chunks == 0ull) return;
     const int pos = tiles[2 * tile + 1] + lane;
@@ -1226,23 +1289,16 @@ chain_visibility_seg_kernel(SceneView s, wc_solve q,
                        wave_min(live ? rx.z : INFINITY)};
     const V3<float> hi{wave_max(live ? rx.x : -INFINITY), wave_max(live ? rx.y : -INFINITY),
                        wave_max(live ? rx.z : -INFINITY)};
+    const unsigned tile_word =
+        cull_segment(s, q, t, base + seg * seg_words * 32, end, sword, found[threadIdx.x >> 6], lo, hi);
+    chunks = __ballot(tile_word != 0u);
     int d = 1;
     while (chunks) {
         const int b = __ffsll((long long)chunks) - 1;
         chunks &= chunks - 1;
-        const int chunk = seg * 64 + b;
-        const unsigned kept = (unsigned)__shfl((int)sword, b);
+        const int chunk = seg * seg_words + b;
         const int c0 = base + chunk * 32;
-        const int c1 = min(c0 + 32, end);
-        bool reach = false;
-        if (lane < c1 - c0 && ((kept >> lane) & 1u)) {
-            const int c = c0 + lane;
-            int dd = 1;
-            while (c >= q.chain_offset[t * kMaxDepth + dd]) ++dd;
-            reach = chain_reaches_box(s, q, c, dd, lo, hi);
-        }
-        unsigned todo = (unsigned)__ballot(reach);
-        if (todo == 0u) continue;
+        unsigned todo = (unsigned)__shfl((int)tile_word, b);
         unsigned bits = 0;
         while (todo) {
             const int bb = __ffs(todo) - 1;
@@ -2463,11 +2519,13 @@ static void launch_chain_visibility(const SceneView& s, const wc_solve& q, const
             hipLaunchKernelGGL(super_cull_kernel, grid, dim3(256), 0, st, s, qs, tiles, supers, words, boxes, sm, base);
         });
         super_masks = sm;
-        if (coherent_tiles(q))
-            for_wave_chunks((long long)tile_count * ((words + 63) / 64), [&](dim3 grid, long long base) {
+        if (coherent_tiles(q)) {
+            const int seg = segment_words(tile_count, words);
+            for_wave_chunks((long long)tile_count * ((words + seg - 1) / seg), [&](dim3 grid, long long base) {
                 hipLaunchKernelGGL(chain_visibility_seg_kernel, grid, dim3(256), 0, st, s, qs, tiles, tile_count,
-                                   masks, words, super_masks, base, touched);
+                                   masks, words, super_masks, base, touched, seg);
             });
+        }
         else
             for_wave_chunks((long long)tile_count * ((words + 63) / 64), [&](dim3 grid, long long base) {
                 hipLaunchKernelGGL(chain_visibility_seg_queue_kernel, grid, dim3(256), 0, st, s, qs, tiles,

@@ -431,8 +431,9 @@ int wc_paths_emit(const wc_scene* scene, const wc_solve* solve, const int* row_o
  * them), instead of testing every candidate of a cell in one lane, twice.
  * `workspace` (wc_paths_masks_workspace_bytes) carries the masks from the
  * count to the emit. path_count also counts visible edges whose field falls
- * below the gain floor; the emit writes such a row with path_length_m NaN,
- * which the canonical compaction drops. row_list: scratch of total + 2 ints,
+ * below the gain floor; the emit writes such a row, and any whose candidate it
+ * does not find again, with path_length_m NaN, which the canonical compaction
+ * drops. row_list: scratch of total + 2 ints,
  * total = the sum of path_count. Rows kept by the compaction are those of
  * wc_paths_count / wc_paths_emit, in the same order. */
 size_t wc_paths_masks_workspace_bytes(int cells, int lanes_per_cell, int edge_count, int max_tx_chains, int tx_count);

@@ -2272,6 +2272,16 @@ __global__ void __launch_bounds__(256) export_diff_kernel(SceneView s, wc_solve 
     write_row(rows, row, ends.t, ends.rx_id, rec);
 }
 
+// A dealt row that turns out to have no path (its length is NaN): its
+// interactions are -1, so it shares no real row's identity and the compaction
+// drops it alone.
+__device__ __forceinline__ void absent_record(int component, int depth, PathRecord& rec) {
+    rec.component = component;
+    rec.depth = depth;
+    rec.edge = -1;
+    for (int j = 0; j < kMaxDepth; ++j) rec.prim[j] = rec.mat[j] = -1;
+}
+
 template <int D>
 __device__ __forceinline__ bool export_chain(const SceneView& s, const wc_solve& q, const RowEnds& ends, int c,
                                              float freq, double k_d, PathRecord& rec) {
@@ -2310,15 +2320,22 @@ __global__ void __launch_bounds__(256) export_main_kernel(SceneView s, wc_solve 
         const V3<float> seg = ends.rx - ends.tx;
         const double dist_d = norm(to_d(ends.rx) - to_d(ends.tx));
         const V3<float> dir = safe_normalize(seg, v3c<float>(0.f, 0.f, 1.f));
-        if (component == kCidLos) {
+        // The walls are gathered again (a few rows per cell block) rather than
+        // kept per cell, and the row follows this gather: whether a segment
+        // meets a wall that it grazes is a matter of rounding, which two kernels
+        // need not share, so the dealt depth does not say how many hits there are.
+        Hit hits[kMaxHits];
+        const int dealt_walls = component == kCidTrans ? rows.primitive_id[row] : 0;
+        const int walls =
+            dealt_walls > 0 ? straight_hits(s, q.components, q.max_depth, ends.tx, seg, dist_d, hits) : 0;
+        if (walls == 0 && (q.components & kCompLos)) {
             los_record(dir, ends.tx_pol, ends.rx_pol, ends.sqrt_power, (float)k_d, k_d, dist_d, rec);
+        } else if (walls >= 1 && walls <= q.max_depth) {
+            transmission_record<true>(s, walls, hits, ends.tx, seg, dir, ends.tx_pol, ends.rx_pol, ends.sqrt_power,
+                                      freq, k_d, dist_d, rec);
         } else {
-            // the walls are gathered again (a few rows per cell block) rather than kept per cell
-            Hit hits[kMaxHits];
-            const int d = rows.primitive_id[row];
-            straight_hits(s, q.components, q.max_depth, ends.tx, seg, dist_d, hits);
-            transmission_record<true>(s, d, hits, ends.tx, seg, dir, ends.tx_pol, ends.rx_pol, ends.sqrt_power, freq,
-                                      k_d, dist_d, rec);
+            ok = false;
+            absent_record(kCidTrans, dealt_walls, rec);
         }
     }
     if (!ok) rec.length = NAN;

@@ -6,6 +6,9 @@
 // Straight rows: a segment through `found` walls dealt as `dealt` walls must be
 // the row of a segment dealt `found` walls (a line-of-sight row without walls),
 // and absent (length NaN, interactions -1) where no such row exists.
+// Chains: a chain of 1 to 5 bounces whose last hit lies off the wall is absent
+// too; with all zeros for its interactions it would carry the identity of a
+// reflection off face 0, and the compaction would drop a real one with it.
 // Input directory: nodes.bin, tris.bin (leaf order), ftris.bin (face order),
 // plane.bin, goff.bin, gfaces.bin of three parallel walls at x = 10, 20, 30.
 // Prints one summary line.
@@ -124,6 +127,36 @@ int main(int argc, char** argv) {
                         wrong += !got.absent(kCidTrans);
                     }
                 }
-    std::printf("straight %ld gone %ld straight_wrong %ld\n", straight, gone, wrong);
+
+    // bounces between walls 0 and 1: wall 0 last, hit on it (y = 4) or off it (y = 400)
+    std::vector<int> chain_groups(kMaxDepth * kMaxDepth, -1), chain_offset(kMaxDepth + 1);
+    std::vector<double> images((size_t)kMaxDepth * kMaxDepth * 3, 0.0);
+    for (int c = 0; c < kMaxDepth; ++c) {
+        chain_offset[c + 1] = c + 1;
+        V3<double> p{15.0, 2.0, 3.0};
+        for (int b = 0; b <= c; ++b) {
+            const int g = (c - b) % 2;
+            chain_groups[c * kMaxDepth + b] = g;
+            double off;
+            const V3<double> n = group_normal(s, g, off);
+            p = p - n * (2.0 * (dot(p, n) - off));
+            double* im = &images[(size_t)(c * kMaxDepth + b) * 3];
+            im[0] = p.x; im[1] = p.y; im[2] = p.z;
+        }
+    }
+    const float between[3] = {15.0f, 2.0f, 3.0f};
+    q.tx_pos = between; q.components = kCompRefl; q.max_depth = kMaxDepth; q.max_tx_chains = kMaxDepth;
+    q.chain_offset = chain_offset.data(); q.chain_groups = chain_groups.data(); q.chain_images = images.data();
+    long chains = 0, kept = 0;
+    for (int c = 0; c < kMaxDepth; ++c)
+        for (const float y : {4.0f, 400.0f}) {
+            rx[0] = 16.0f;
+            rx[1] = y;
+            const Row got = evaluate(s, q, kCidRefl, c);
+            ++chains;
+            if (y < 40.0f) kept += got.component == kCidRefl && got.depth == c + 1 && got.length > 0.0f && got.seq[0] >= 0;
+            else kept += got.absent(kCidRefl) && got.depth == c + 1;
+        }
+    std::printf("chains %ld chains_right %ld straight %ld gone %ld straight_wrong %ld\n", chains, kept, straight, gone, wrong);
     return 0;
 }

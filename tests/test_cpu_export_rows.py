@@ -43,3 +43,7 @@ def report(tmp_path_factory):
 def test_straight_row_follows_the_walls_its_kernel_finds(report):
     assert report["straight"] == 120 and report["gone"] > 0
     assert report["straight_wrong"] == 0
+
+
+def test_chain_without_hits_leaves_an_absent_row(report):
+    assert report["chains"] == report["chains_right"] == 10

@@ -132,3 +132,23 @@ def test_pair_order_and_row_offsets_match_numpy(device, seed):
     starts[want] = scan[:-1]
     assert np.array_equal(row_offset.cpu().numpy(), starts)
     assert int(total.item()) == int(counts.sum())
+
+
+def test_absent_row_drops_alone(device):
+    """A reflection row without a path (length NaN, interactions -1) beside a
+    reflection off face 0 of the same depth: only the absent one goes."""
+    rows = {"depth": np.array([1, 1, 2, 2], np.int32), "component_id": np.ones(4, np.int32),
+            "primitive_sequence": np.array([[0, -1], [-1, -1], [-1, -1], [0, 0]], np.int32),
+            "primitive_id": np.array([0, -1, -1, 0], np.int32), "edge_id": np.full(4, -1, np.int32),
+            "path_length_m": np.array([5.0, np.nan, np.nan, 7.0], np.float32)}
+    assert oracle.canonical_compact(rows, np.array([0, 4]))["source_row"].tolist() == [0, 3]
+    view, keep_alive = _device_rows(rows, device)
+    p = _native.ptr
+    offset = torch.tensor([0, 4], dtype=torch.int32, device=device)
+    perm = torch.empty(4, dtype=torch.int32, device=device)
+    keep = torch.empty(4, dtype=torch.uint8, device=device)
+    _native.call("wc_paths_canonical_order", ctypes.byref(view), p(offset), 1, p(perm), p(keep),
+                 _native.stream_handle(device))
+    kept = perm[keep.bool()].tolist()
+    assert kept == [0, 3]
+    del keep_alive

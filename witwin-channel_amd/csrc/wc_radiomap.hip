@@ -2312,10 +2312,7 @@ __global__ void __launch_bounds__(256) export_main_kernel(SceneView s, wc_solve 
             case 4: ok = export_chain<4>(s, q, ends, c, freq, k_d, rec); break;
             default: ok = export_chain<5>(s, q, ends, c, freq, k_d, rec); break;
         }
-        if (!ok) {
-            rec.component = kCidRefl;
-            rec.depth = d;
-        }
+        if (!ok) absent_record(kCidRefl, d, rec);
     } else {
         const V3<float> seg = ends.rx - ends.tx;
         const double dist_d = norm(to_d(ends.rx) - to_d(ends.tx));

@@ -66,20 +66,24 @@ int wc_bvh_build_sah(const float* vertices_host, const int* faces_host, const in
  * wc_edge_candidates: the edges one or two faces share, in order of first
  * appearance over the face edges (f, k). Replaces the per-edge host tables of
  * the reference's scene/resources.py:79-148, 286-404.
- *   welded [V,3]: vertex positions in weld steps; faces [F,3];
+ *   welded [V,3]: vertex positions in weld steps; faces [F,3] (vertex ids, from
+ *   the end where negative; an id outside the V vertices is refused);
  *   face_structure [F], structure_vertex_base [S]: owner of each face and the
  *   first vertex of each structure; face_group / face_material [F]
  *   vertex_ids [3F,4] (a, b, c0, c1 or -1), face_ids [3F,6] (face0, face1,
  *   group0, group1, material0, material1; -1 without a second face),
  *   public_ids [3F]: room for every face edge; *count: candidates written.
- * wc_group_hulls: convex hull of every coplanar group in its plane,
- *   hull_offset [G+1], hull_points [2 * 3 * listed faces, 3]. */
-int wc_edge_candidates(const long long* welded, const int* faces, int face_count, const long long* face_structure,
-                       const long long* structure_vertex_base, int structure_count, const int* face_group,
-                       const int* face_material, long long* vertex_ids, long long* face_ids, long long* public_ids,
-                       int* count);
-int wc_group_hulls(const float* vertices, const int* faces, const int* group_face_offset, const int* group_faces,
-                   const double* group_plane, int group_count, int* hull_offset, double* hull_points);
+ * wc_group_hulls: convex hull of every coplanar group in its plane, group g
+ *   being faces group_faces[group_face_offset[g] .. group_face_offset[g+1]) of
+ *   listed_count; hull_offset [G+1], hull_points [2 * 3 * listed_count, 3].
+ *   Offsets, faces and vertices outside their arrays are refused. */
+int wc_edge_candidates(const long long* welded, int vertex_count, const int* faces, int face_count,
+                       const long long* face_structure, const long long* structure_vertex_base, int structure_count,
+                       const int* face_group, const int* face_material, long long* vertex_ids, long long* face_ids,
+                       long long* public_ids, int* count);
+int wc_group_hulls(const float* vertices, int vertex_count, const int* faces, int face_count,
+                   const int* group_face_offset, const int* group_faces, int listed_count, const double* group_plane,
+                   int group_count, int* hull_offset, double* hull_points);
 /* Collapse of a binary tree (wc_bvh_build's nodes, copied to the host) into
  * the 4-wide nodes of the scene view: each wide node takes a binary node's
  * children and opens the internal child of largest surface area until it

@@ -76,6 +76,81 @@ def test_edge_candidates_refuse_an_unknown_structure():
                                   structure_vertex_base=base)
 
 
+@pytest.mark.parametrize("vertex", [23, 2 ** 32, -24])
+def test_faces_outside_the_vertices_are_refused(vertex):
+    vertices, faces, _, _ = _random_mesh(1)
+    assert len(vertices) == 23
+    faces = faces.astype(np.int64)
+    faces[-1, 2] = vertex
+    n = len(faces)
+    with pytest.raises(IndexError):
+        compiler.build_edge_table(vertices, faces, np.arange(n), np.zeros(n, np.int32))
+    with pytest.raises(IndexError):
+        compiler.group_hulls(vertices, faces, np.arange(n + 1), np.arange(n), np.tile([0.0, 0.0, 1.0, 0.0], (n, 1)))
+
+
+def test_short_tables_are_refused():
+    vertices, faces, structure, base = _random_mesh(1)
+    n = len(faces)
+    group, material = np.arange(n), np.zeros(n, np.int32)
+    for tables in ((group[:-1], material, structure), (group, material[:-1], structure),
+                   (group, material, structure[:-1])):
+        with pytest.raises(IndexError):
+            compiler.build_edge_table(vertices, faces, tables[0], tables[1], face_structure=tables[2],
+                                      structure_vertex_base=base)
+    plane = np.tile([0.0, 0.0, 1.0, 0.0], (n, 1))
+    for offset, listed in ((np.arange(n), np.arange(n)), (np.arange(n + 1), np.arange(1, n + 1))):
+        with pytest.raises(IndexError):
+            compiler.group_hulls(vertices, faces, offset, listed, plane)
+    with pytest.raises(RuntimeError, match="group"):
+        compiler.group_hulls(vertices, faces, np.arange(n + 1), np.arange(n - 1), plane)
+
+
+def test_native_entries_refuse_indices_outside_their_arrays():
+    """The C entry points themselves, as a caller without the Python checks."""
+    from witwin.channel import _native
+
+    welded, v = np.zeros((3, 3), np.int64), np.eye(3, dtype=np.float32)
+    zeros, base = np.zeros(1, np.int64), np.zeros(1, np.int64)
+    ids = [np.zeros((3, k), np.int64) for k in (4, 6, 1)]
+    count, offset, plane = np.zeros(1, np.int32), np.zeros(2, np.int32), np.array([[0.0, 0.0, 1.0, 0.0]])
+    table, points = np.zeros(1, np.int32), np.zeros((6, 3))
+
+    def edges(face):
+        tri = np.array([face], np.int32)
+        _native.call("wc_edge_candidates", welded.ctypes.data, 3, tri.ctypes.data, 1, zeros.ctypes.data,
+                     base.ctypes.data, 1, table.ctypes.data, table.ctypes.data, *(a.ctypes.data for a in ids),
+                     count.ctypes.data)
+
+    def hulls(face, first=(0, 1), listed=(0,)):
+        tri, first, listed = (np.array(a, np.int32) for a in ([face], first, listed))
+        _native.call("wc_group_hulls", v.ctypes.data, 3, tri.ctypes.data, 1, first.ctypes.data, listed.ctypes.data,
+                     len(listed), plane.ctypes.data, 1, offset.ctypes.data, points.ctypes.data)
+
+    edges([0, 1, 2])
+    hulls([0, 1, 2])
+    assert offset.tolist() == [0, 3]
+    for face in ([0, 1, 3], [0, -4, 2]):
+        with pytest.raises(RuntimeError, match="vertex"):
+            edges(face)
+        with pytest.raises(RuntimeError, match="vertex"):
+            hulls(face)
+    for first, listed in (((0, 2), (0,)), ((1, 0), (0,)), ((-1, 1), (0,))):
+        with pytest.raises(RuntimeError, match="group"):
+            hulls([0, 1, 2], first, listed)
+    with pytest.raises(RuntimeError, match="face"):
+        hulls([0, 1, 2], (0, 1), (1,))
+
+
+def test_negative_face_and_vertex_ids_count_from_the_end():
+    vertices, faces, _, _ = _random_mesh(2)
+    n = len(faces)
+    plane = np.tile([0.0, 0.6, 0.8, 0.3], (n, 1))
+    a = compiler.group_hulls(vertices, faces, np.arange(n + 1), np.arange(n), plane)
+    b = compiler.group_hulls(vertices, faces - len(vertices), np.arange(n + 1), np.arange(n) - n, plane)
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+
+
 def test_empty_mesh():
     none = np.zeros((0, 3), np.int32)
     edges, ev = compiler.build_edge_table(np.zeros((0, 3), np.float32), none, np.zeros(0, np.int32),

@@ -39,6 +39,12 @@ struct P2 {
     double x, y;
 };
 
+// A host array's index, from its end where negative; -1 outside the array.
+int64_t array_index(int64_t i, int64_t count) {
+    if (i < 0) i += count;
+    return i >= 0 && i < count ? i : -1;
+}
+
 // hull of points sorted by (x, y), as the monotone chain builds one side
 void half_hull(const std::vector<P2>& seq, std::vector<P2>& out) {
     out.clear();
@@ -57,11 +63,12 @@ void half_hull(const std::vector<P2>& seq, std::vector<P2>& out) {
 
 using namespace wc;
 
-extern "C" int wc_edge_candidates(const long long* welded, const int* faces, int face_count,
+extern "C" int wc_edge_candidates(const long long* welded, int vertex_count, const int* faces, int face_count,
                                   const long long* face_structure, const long long* structure_vertex_base,
                                   int structure_count, const int* face_group, const int* face_material,
                                   long long* vertex_ids, long long* face_ids, long long* public_ids, int* count) {
-    if (face_count < 0 || structure_count < 0) return wc_fail("wc_edge_candidates: sizes must be non-negative");
+    if (vertex_count < 0 || face_count < 0 || structure_count < 0)
+        return wc_fail("wc_edge_candidates: sizes must be non-negative");
     if (!count) return wc_fail("wc_edge_candidates: count is null");
     *count = 0;
     if (face_count == 0) return 0;
@@ -75,6 +82,9 @@ extern "C" int wc_edge_candidates(const long long* welded, const int* faces, int
             if (face_structure[f] < 0 || face_structure[f] >= structure_count)
                 return wc_fail("wc_edge_candidates: face %d belongs to structure %lld of %d", f, face_structure[f],
                                structure_count);
+        for (int i = 0; i < n; ++i)
+            if (array_index(faces[i], vertex_count) < 0)
+                return wc_fail("wc_edge_candidates: face %d names vertex %d of %d", i / 3, faces[i], vertex_count);
         auto corner = [&](int e, int k) { return faces[3 * (e / 3) + (e % 3 + k) % 3]; };
         // public id of a face edge: the rank of its (structure, lower, higher local vertex) among the distinct ones
         struct Record {
@@ -104,7 +114,8 @@ extern "C" int wc_edge_candidates(const long long* welded, const int* faces, int
         std::vector<EdgeEntry> entries;
         entries.reserve((size_t)n);
         for (int e = 0; e < n; ++e) {
-            const long long *a = welded + 3 * (size_t)corner(e, 0), *b = welded + 3 * (size_t)corner(e, 1);
+            const long long *a = welded + 3 * array_index(corner(e, 0), vertex_count),
+                            *b = welded + 3 * array_index(corner(e, 1), vertex_count);
             if (std::lexicographical_compare(b, b + 3, a, a + 3)) std::swap(a, b);
             EdgeKey key;
             for (int k = 0; k < 3; ++k) {
@@ -149,14 +160,28 @@ extern "C" int wc_edge_candidates(const long long* welded, const int* faces, int
     return 0;
 }
 
-extern "C" int wc_group_hulls(const float* vertices, const int* faces, const int* group_face_offset,
-                              const int* group_faces, const double* group_plane, int group_count, int* hull_offset,
-                              double* hull_points) {
-    if (group_count < 0 || !hull_offset) return wc_fail("wc_group_hulls: invalid arguments");
+extern "C" int wc_group_hulls(const float* vertices, int vertex_count, const int* faces, int face_count,
+                              const int* group_face_offset, const int* group_faces, int listed_count,
+                              const double* group_plane, int group_count, int* hull_offset, double* hull_points) {
+    if (vertex_count < 0 || face_count < 0 || listed_count < 0 || group_count < 0 || !hull_offset)
+        return wc_fail("wc_group_hulls: invalid arguments");
     hull_offset[0] = 0;
     if (group_count == 0) return 0;
     if (!vertices || !faces || !group_face_offset || !group_faces || !group_plane || !hull_points)
         return wc_fail("wc_group_hulls: null argument");
+    for (int g = 0; g < group_count; ++g)
+        if (group_face_offset[g] < 0 || group_face_offset[g] > group_face_offset[g + 1] ||
+            group_face_offset[g + 1] > listed_count)
+            return wc_fail("wc_group_hulls: group %d lists faces %d to %d of %d", g, group_face_offset[g],
+                           group_face_offset[g + 1], listed_count);
+    for (int i = group_face_offset[0]; i < group_face_offset[group_count]; ++i) {
+        const int64_t f = array_index(group_faces[i], face_count);
+        if (f < 0) return wc_fail("wc_group_hulls: face %d of %d is listed", group_faces[i], face_count);
+        for (int k = 0; k < 3; ++k)
+            if (array_index(faces[3 * f + k], vertex_count) < 0)
+                return wc_fail("wc_group_hulls: face %lld names vertex %d of %d", (long long)f, faces[3 * f + k],
+                               vertex_count);
+    }
     try {
         std::vector<P2> pts, rev, lower, upper;
         size_t total = 0;
@@ -176,14 +201,16 @@ extern "C" int wc_group_hulls(const float* vertices, const int* faces, const int
             const int begin = group_face_offset[g], end = group_face_offset[g + 1];
             pts.clear();
             bool finite = true;
-            for (int i = begin; i < end; ++i)
+            for (int i = begin; i < end; ++i) {
+                const int* face = faces + 3 * array_index(group_faces[i], face_count);
                 for (int k = 0; k < 3; ++k) {
-                    const float* p = vertices + 3 * (size_t)faces[3 * (size_t)group_faces[i] + k];
+                    const float* p = vertices + 3 * array_index(face[k], vertex_count);
                     const double d[3] = {p[0] - o[0], p[1] - o[1], p[2] - o[2]};
                     const P2 q{d[0] * u[0] + d[1] * u[1] + d[2] * u[2], d[0] * w[0] + d[1] * w[1] + d[2] * w[2]};
                     finite = finite && std::isfinite(q.x) && std::isfinite(q.y);
                     pts.push_back(q);
                 }
+            }
             if (end - begin == 1) {
                 const double area = (pts[1].x - pts[0].x) * (pts[2].y - pts[0].y) -
                                     (pts[1].y - pts[0].y) * (pts[2].x - pts[0].x);

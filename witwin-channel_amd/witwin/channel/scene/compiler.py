@@ -295,6 +295,15 @@ def _edge_rows(geometry: dict[str, np.ndarray], ids: np.ndarray) -> np.ndarray:
     return rows
 
 
+def _check_faces(faces: np.ndarray, vertex_count: int) -> None:
+    """IndexError for a face whose vertex ids are not the array's (as indexing
+    the array raises it), before they are narrowed and handed to native code."""
+    if faces.ndim != 2 or faces.shape[1] != 3:
+        raise IndexError(f"faces must be [F, 3], got {tuple(faces.shape)}")
+    if faces.size and (int(faces.max()) >= vertex_count or int(faces.min()) < -vertex_count):
+        raise IndexError(f"faces name vertices {int(faces.min())} to {int(faces.max())} of {vertex_count}")
+
+
 def build_edge_table(vertices: np.ndarray, faces: np.ndarray, face_group: np.ndarray, face_material: np.ndarray,
                      policy: str = "all", face_structure: np.ndarray | None = None,
                      structure_vertex_base: np.ndarray | None = None,
@@ -327,15 +336,19 @@ def build_edge_table(vertices: np.ndarray, faces: np.ndarray, face_group: np.nda
     v = vertices.astype(np.float64)
     q = np.ascontiguousarray(np.rint(v / EDGE_WELD_QUANTIZATION).astype(np.int64))
     n_faces = int(faces.shape[0])
+    _check_faces(np.asarray(faces), int(q.shape[0]))
     host = lambda x, dt: np.ascontiguousarray(x, dtype=dt)  # noqa: E731
     tri, group, material = host(faces, np.int32), host(face_group, np.int32), host(face_material, np.int32)
     fstruct = np.zeros(n_faces, np.int64) if face_structure is None else host(face_structure, np.int64)
     vbase = np.zeros(1, np.int64) if structure_vertex_base is None else host(structure_vertex_base, np.int64)
+    if group.shape[0] < n_faces or material.shape[0] < n_faces or fstruct.shape[0] != n_faces:
+        raise IndexError(f"{n_faces} faces with {group.shape[0]} groups, {material.shape[0]} materials and "
+                         f"{fstruct.shape[0]} structures")
     ev = np.empty((3 * n_faces, 4), np.int64)
     ids = np.empty((3 * n_faces, 6), np.int64)
     pid = np.empty(3 * n_faces, np.int64)
     count = np.zeros(1, np.int32)
-    _native.call("wc_edge_candidates", q.ctypes.data, tri.ctypes.data, n_faces, fstruct.ctypes.data,
+    _native.call("wc_edge_candidates", q.ctypes.data, int(q.shape[0]), tri.ctypes.data, n_faces, fstruct.ctypes.data,
                  vbase.ctypes.data, int(vbase.shape[0]), group.ctypes.data, material.ctypes.data, ev.ctypes.data,
                  ids.ctypes.data, pid.ctypes.data, count.ctypes.data)
     ev, ids, pid = (x[:int(count[0])] for x in (ev, ids, pid))
@@ -549,10 +562,16 @@ def group_hulls(vertices: np.ndarray, faces: np.ndarray, group_face_offset: np.n
     g = int(group_plane.shape[0])
     verts, tri, plane = host(vertices, np.float32), host(faces, np.int32), host(group_plane, np.float64)
     first, members = host(group_face_offset, np.int32), host(group_faces, np.int32)
+    _check_faces(np.asarray(faces), int(verts.shape[0]))
+    if members.size and (int(members.max()) >= tri.shape[0] or int(members.min()) < -tri.shape[0]):
+        raise IndexError(f"groups list faces {int(members.min())} to {int(members.max())} of {tri.shape[0]}")
+    if first.shape[0] != g + 1:
+        raise IndexError(f"{g} groups with {first.shape[0]} face offsets")
     offset = np.zeros(g + 1, np.int32)
     points = np.empty((3 * int(members.shape[0]) * 2, 3), np.float64)
-    _native.call("wc_group_hulls", verts.ctypes.data, tri.ctypes.data, first.ctypes.data, members.ctypes.data,
-                 plane.ctypes.data, g, offset.ctypes.data, points.ctypes.data)
+    _native.call("wc_group_hulls", verts.ctypes.data, int(verts.shape[0]), tri.ctypes.data, int(tri.shape[0]),
+                 first.ctypes.data, members.ctypes.data, int(members.shape[0]), plane.ctypes.data, g,
+                 offset.ctypes.data, points.ctypes.data)
     return offset, np.ascontiguousarray(points[:int(offset[g])])
 
 

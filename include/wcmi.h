@@ -81,7 +81,7 @@ int wc_edge_candidates(const long long* welded, int vertex_count, const int* fac
                        const long long* face_structure, const long long* structure_vertex_base, int structure_count,
                        const int* face_group, const int* face_material, long long* vertex_ids, long long* face_ids,
                        long long* public_ids, int* count);
-int wc_group_hulls(const float* vertices, int vertex_count, const int* faces, int face_count,
+int wc_group_hulls(const double* vertices, int vertex_count, const int* faces, int face_count,
                    const int* group_face_offset, const int* group_faces, int listed_count, const double* group_plane,
                    int group_count, int* hull_offset, double* hull_points);
 /* Collapse of a binary tree (wc_bvh_build's nodes, copied to the host) into

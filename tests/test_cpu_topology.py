@@ -110,7 +110,7 @@ def test_native_entries_refuse_indices_outside_their_arrays():
     """The C entry points themselves, as a caller without the Python checks."""
     from witwin.channel import _native
 
-    welded, v = np.zeros((3, 3), np.int64), np.eye(3, dtype=np.float32)
+    welded, v = np.zeros((3, 3), np.int64), np.eye(3)
     zeros, base = np.zeros(1, np.int64), np.zeros(1, np.int64)
     ids = [np.zeros((3, k), np.int64) for k in (4, 6, 1)]
     count, offset, plane = np.zeros(1, np.int32), np.zeros(2, np.int32), np.array([[0.0, 0.0, 1.0, 0.0]])
@@ -159,6 +159,18 @@ def test_empty_mesh():
     offset, points = compiler.group_hulls(np.zeros((0, 3), np.float32), none, np.zeros(1, np.int32),
                                           np.zeros(0, np.int32), np.zeros((0, 4)))
     assert offset.tolist() == [0] and points.shape == (0, 3)
+
+
+def test_group_hulls_keep_float64_vertices():
+    """Corners are the vertices given: a few roundings of the in-plane basis on
+    coordinates below 10 (1e-14), where single precision would move them 5e-7."""
+    vertices = np.random.default_rng(3).uniform(-5.0, 5.0, (3, 3))
+    n = np.cross(vertices[1] - vertices[0], vertices[2] - vertices[0])
+    n /= np.linalg.norm(n)
+    offset, points = compiler.group_hulls(vertices, np.array([[0, 1, 2]]), np.array([0, 1]), np.array([0]),
+                                          np.append(n, n @ vertices[0])[None])
+    assert offset.tolist() == [0, 3]
+    assert np.abs(points[:, None] - vertices[None]).max(axis=2).min(axis=1).max() < 1e-14
 
 
 def test_group_hulls_contain_their_faces():

@@ -160,7 +160,7 @@ extern "C" int wc_edge_candidates(const long long* welded, int vertex_count, con
     return 0;
 }
 
-extern "C" int wc_group_hulls(const float* vertices, int vertex_count, const int* faces, int face_count,
+extern "C" int wc_group_hulls(const double* vertices, int vertex_count, const int* faces, int face_count,
                               const int* group_face_offset, const int* group_faces, int listed_count,
                               const double* group_plane, int group_count, int* hull_offset, double* hull_points) {
     if (vertex_count < 0 || face_count < 0 || listed_count < 0 || group_count < 0 || !hull_offset)
@@ -204,7 +204,7 @@ extern "C" int wc_group_hulls(const float* vertices, int vertex_count, const int
             for (int i = begin; i < end; ++i) {
                 const int* face = faces + 3 * array_index(group_faces[i], face_count);
                 for (int k = 0; k < 3; ++k) {
-                    const float* p = vertices + 3 * array_index(face[k], vertex_count);
+                    const double* p = vertices + 3 * array_index(face[k], vertex_count);
                     const double d[3] = {p[0] - o[0], p[1] - o[1], p[2] - o[2]};
                     const P2 q{d[0] * u[0] + d[1] * u[1] + d[2] * u[2], d[0] * w[0] + d[1] * w[1] + d[2] * w[2]};
                     finite = finite && std::isfinite(q.x) && std::isfinite(q.y);

@@ -560,7 +560,7 @@ def group_hulls(vertices: np.ndarray, faces: np.ndarray, group_face_offset: np.n
 
     host = lambda x, dt: np.ascontiguousarray(x, dtype=dt)  # noqa: E731
     g = int(group_plane.shape[0])
-    verts, tri, plane = host(vertices, np.float32), host(faces, np.int32), host(group_plane, np.float64)
+    verts, tri, plane = host(vertices, np.float64), host(faces, np.int32), host(group_plane, np.float64)
     first, members = host(group_face_offset, np.int32), host(group_faces, np.int32)
     _check_faces(np.asarray(faces), int(verts.shape[0]))
     if members.size and (int(members.max()) >= tri.shape[0] or int(members.min()) < -tri.shape[0]):

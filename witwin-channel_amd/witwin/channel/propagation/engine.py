@@ -631,9 +631,15 @@ def pair_order(dscene: DeviceScene, inputs: SolveInputs) -> torch.Tensor:
 # The masked export holds one bit per (cell, chain) and per (cell, edge). Above
 # this many bytes it would crowd the rows themselves out of memory, and the
 # per-cell kernels, which need none, do the export (as they do when the masks
-# cannot be allocated). Both write the same rows; on 45,221 pairs with 0.8 M
-# rows the batched solve takes 3.3 ms with the masks and 57.3 ms per cell.
+# cannot be allocated). Both keep the same rows; the masked one emits visible
+# edges below the gain floor too and leaves them to the compaction. On 45,221
+# pairs with 0.8 M rows the batched solve takes 3.3 ms with the masks and
+# 57.3 ms per cell.
 EXPORT_MASK_LIMIT = 16 << 30
+
+
+class RowLimitError(RuntimeError):
+    """More emitted rows than the row index holds."""
 
 
 def export_masks(dscene: DeviceScene, inputs: SolveInputs) -> torch.Tensor | None:
@@ -661,12 +667,27 @@ def export_rows(dscene: DeviceScene, inputs: SolveInputs, *, width: int,
     canonical pair) describe the kept rows' segmentation; ``dropped`` counts
     identity winners removed by the cap."""
 
+    held = [export_masks(dscene, inputs)]
+    if held[0] is not None:
+        # the masked export takes more memory than the per-cell one (its masks,
+        # and rows below the gain floor): where it does not fit, that one may
+        try:
+            return _export_rows(dscene, inputs, width, max_paths_per_pair, held)
+        except (torch.OutOfMemoryError, RowLimitError):
+            held.clear()
+    return _export_rows(dscene, inputs, width, max_paths_per_pair, [None])
+
+
+def _export_rows(dscene: DeviceScene, inputs: SolveInputs, width: int, max_paths_per_pair: int | None,
+                 held: list[torch.Tensor | None]) -> dict[str, Any]:
+    """export_rows on the masks in ``held`` (taken out of it and released once
+    the rows are written), or per cell where it holds None."""
     device = dscene.device
     cells = inputs.total_cells
     stream = _native.stream_handle(device)
     p = _native.ptr
     counts = torch.empty(max(cells, 1), dtype=torch.int32, device=device)
-    masks = export_masks(dscene, inputs)
+    masks = held.pop()
     if masks is not None:
         _native.call("wc_paths_count_masked", dscene.ref(), ctypes.byref(inputs.view), p(masks), p(inputs.tiles),
                      inputs.tile_count, p(counts), stream)
@@ -682,7 +703,7 @@ def export_rows(dscene: DeviceScene, inputs: SolveInputs, *, width: int,
                  p(totals), p(ws), stream)
     total = int(totals[0].item())
     if total >= 2 ** 31:
-        raise RuntimeError(f"path export: {total} rows exceed the int32 row index")
+        raise RowLimitError(f"path export: {total} rows exceed the int32 row index")
     w = max(int(width), 1)
     k = max(total, 1)
     rows: dict[str, torch.Tensor] = {}
@@ -707,9 +728,11 @@ def export_rows(dscene: DeviceScene, inputs: SolveInputs, *, width: int,
         row_list = torch.empty(total + 2, dtype=torch.int32, device=device)
         _native.call("wc_paths_emit_masked", dscene.ref(), ctypes.byref(inputs.view), p(masks), p(inputs.tiles),
                      inputs.tile_count, p(row_offset), p(counts), total, p(row_list), ctypes.byref(view), stream)
+        del row_list
     elif total:
         _native.call("wc_paths_emit", dscene.ref(), ctypes.byref(inputs.view), p(row_offset), p(counts),
                      ctypes.byref(view), stream)
+    del masks
     perm = torch.empty(k, dtype=torch.int32, device=device)
     keep = torch.empty(k, dtype=torch.uint8, device=device)
     kept_offset = torch.empty(cells + 1, dtype=torch.int32, device=device)

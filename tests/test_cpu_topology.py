@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import numpy as np
 import pytest
+import torch
 
 from witwin.channel import workloads
 from witwin.channel.scene import compiler
@@ -187,3 +188,14 @@ def test_group_hulls_contain_their_faces():
         assert np.abs(hull[:, None] - pts[None]).max(axis=2).min(axis=1).max() < 1e-4  # off-plane part of a vertex
         for a, b in zip(hull, np.roll(hull, -1, axis=0)):
             assert (np.cross(b - a, pts - a) @ n >= -1e-9 * np.linalg.norm(b - a) * 400.0).all()
+
+
+def test_scene_tables_count_their_own_changes():
+    c = compiler.compile(workloads.urban_canyon_scene(seed=2, shape=(2, 2)), reference_frequency_hz=3.5e9)
+    scene = compiler.DeviceScene(c, torch.device("cpu"))
+    x = torch.ones(1, requires_grad=True)
+    y = (x * scene.mat_eps).sum()
+    scene.vertices.add_(1.0)
+    y.backward()
+    assert x.grad.item() == pytest.approx(float(scene.mat_eps.sum()))
+    assert np.array_equal(scene.vertices.numpy(), c.vertices + np.float32(1.0))

@@ -576,8 +576,10 @@ def group_hulls(vertices: np.ndarray, faces: np.ndarray, group_face_offset: np.n
 
 
 def _upload(device: torch.device, arrays: list[tuple[np.ndarray, np.dtype]]) -> list[torch.Tensor]:
-    """Device copies of host arrays as views of one buffer (one transfer;
-    256-byte aligned parts)."""
+    """Device copies of host arrays as parts of one buffer (one transfer;
+    256-byte aligned parts). Each counts its own in-place changes: views of one
+    tensor would share that count, and a refit of the vertices would then refuse
+    the backward pass of a graph that keeps a material table."""
     host = [np.ascontiguousarray(a, dtype=dt) for a, dt in arrays]
     start = np.concatenate([[0], np.cumsum([(a.nbytes + 255) // 256 * 256 for a in host])]).astype(np.int64)
     packed = np.zeros(max(int(start[-1]), 1), np.uint8)
@@ -587,7 +589,7 @@ def _upload(device: torch.device, arrays: list[tuple[np.ndarray, np.dtype]]) -> 
     out = []
     for a, at in zip(host, start):
         dtype = torch.from_numpy(np.empty(0, a.dtype)).dtype
-        out.append(buffer[int(at):int(at) + a.nbytes].view(dtype).reshape(a.shape) if a.nbytes
+        out.append(buffer[int(at):int(at) + a.nbytes].view(dtype).reshape(a.shape).data if a.nbytes
                    else torch.empty(a.shape, dtype=dtype, device=device))
     return out
 

@@ -199,3 +199,15 @@ def test_scene_tables_count_their_own_changes():
     y.backward()
     assert x.grad.item() == pytest.approx(float(scene.mat_eps.sum()))
     assert np.array_equal(scene.vertices.numpy(), c.vertices + np.float32(1.0))
+
+
+def test_scene_hulls_are_those_of_the_uploaded_vertices():
+    """Changing the compiled scene's arrays afterwards moves neither the device
+    tables nor the hulls the chain culls bound their planes with."""
+    c = compiler.compile(workloads.urban_canyon_scene(seed=2, shape=(2, 2)), reference_frequency_hz=3.5e9)
+    want = compiler.DeviceScene(c, torch.device("cpu")).hulls()
+    scene = compiler.DeviceScene(c, torch.device("cpu"))
+    for table in (c.vertices, c.group_plane):
+        table += 5.0
+    for a, b in zip(scene.hulls(), want):
+        assert torch.equal(a, b)

@@ -645,9 +645,11 @@ class DeviceScene:
         self.edge_count = compiled.edge_count
         self._csr: tuple[torch.Tensor, torch.Tensor] | None = None
         self._hulls: tuple[torch.Tensor, torch.Tensor] | None = None
-        # the arrays the group hulls are made of, until a refit moves them
-        self._hull_host = (compiled.vertices, compiled.faces, compiled.group_face_offset, compiled.group_faces,
-                           compiled.group_plane)
+        # what the group hulls are made of, as uploaded (the compiled scene's arrays may change later), until a
+        # refit moves it
+        self._hull_host = tuple(np.array(a, dtype=dt) for a, dt in (
+            (compiled.vertices, f32), (compiled.faces, i32), (compiled.group_face_offset, i32),
+            (compiled.group_faces, i32), (compiled.group_plane, np.float64)))
         wide_host = nodes
         if f and bvh == "lbvh":
             ws_bytes = int(_native.call("wc_bvh_workspace_bytes", f))
@@ -716,6 +718,7 @@ class DeviceScene:
                 self.group_faces.cpu().numpy(), self.group_plane.cpu().numpy())))
             self._hulls = (torch.as_tensor(offset).to(self.device),
                            torch.as_tensor(points if points.size else np.zeros((1, 3))).to(self.device))
+            self._hull_host = None
         return self._hulls
 
     def vertex_csr(self) -> tuple[torch.Tensor, torch.Tensor]:

@@ -1,10 +1,15 @@
-"""The native host part of scene compilation (wc_topology.hip) against plain
+"""The native host part of scene compilation (wc_topology.cpp) against plain
 restatements: edge candidates with their public ids (reference
 scene/resources.py:79-148, 286-404) on meshes with shared, boundary,
 non-manifold, welded-apart and degenerate edges, and the hulls of coplanar
 groups."""
 
 from __future__ import annotations
+
+import os
+import subprocess
+import sys
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -107,10 +112,23 @@ def test_short_tables_are_refused():
         compiler.group_hulls(vertices, faces, np.arange(n + 1), np.arange(n - 1), plane)
 
 
-def test_native_entries_refuse_indices_outside_their_arrays():
+def test_compiling_a_scene_does_not_load_the_gpu_library():
+    """In a process of its own: libwcmi.so, loaded before the GPU runtime, slows
+    every later allocation and launch."""
+    code = ("import torch; from witwin.channel import workloads; from witwin.channel.scene import compiler;"
+            "compiler.compile(workloads.wedge_diffraction_scene(), reference_frequency_hz=3.5e9);"
+            "print('libwcmi.so' in open('/proc/self/maps').read(), 'libwcmi_host.so' in open('/proc/self/maps').read())")
+    run = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300,
+                         env={**os.environ, "PYTHONPATH": str(Path(compiler.__file__).resolve().parents[3])})
+    assert run.stdout.split() == ["False", "True"], run.stdout + run.stderr
+
+
+@pytest.mark.parametrize("call", ["call", "call_host"])
+def test_native_entries_refuse_indices_outside_their_arrays(call):
     """The C entry points themselves, as a caller without the Python checks."""
     from witwin.channel import _native
 
+    native = getattr(_native, call)
     welded, v = np.zeros((3, 3), np.int64), np.eye(3)
     zeros, base = np.zeros(1, np.int64), np.zeros(1, np.int64)
     ids = [np.zeros((3, k), np.int64) for k in (4, 6, 1)]
@@ -119,14 +137,14 @@ def test_native_entries_refuse_indices_outside_their_arrays():
 
     def edges(face):
         tri = np.array([face], np.int32)
-        _native.call("wc_edge_candidates", welded.ctypes.data, 3, tri.ctypes.data, 1, zeros.ctypes.data,
-                     base.ctypes.data, 1, table.ctypes.data, table.ctypes.data, *(a.ctypes.data for a in ids),
-                     count.ctypes.data)
+        native("wc_edge_candidates", welded.ctypes.data, 3, tri.ctypes.data, 1, zeros.ctypes.data,
+               base.ctypes.data, 1, table.ctypes.data, table.ctypes.data, *(a.ctypes.data for a in ids),
+               count.ctypes.data)
 
     def hulls(face, first=(0, 1), listed=(0,)):
         tri, first, listed = (np.array(a, np.int32) for a in ([face], first, listed))
-        _native.call("wc_group_hulls", v.ctypes.data, 3, tri.ctypes.data, 1, first.ctypes.data, listed.ctypes.data,
-                     len(listed), plane.ctypes.data, 1, offset.ctypes.data, points.ctypes.data)
+        native("wc_group_hulls", v.ctypes.data, 3, tri.ctypes.data, 1, first.ctypes.data, listed.ctypes.data,
+               len(listed), plane.ctypes.data, 1, offset.ctypes.data, points.ctypes.data)
 
     edges([0, 1, 2])
     hulls([0, 1, 2])

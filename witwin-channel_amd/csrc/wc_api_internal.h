@@ -2,12 +2,12 @@
 // thread-local message readable through wc_last_error().
 #pragma once
 
+#include "wc_error.h"
+
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <cstddef>
 
-// printf-style message; returns 1
-int wc_fail(const char* format, ...) __attribute__((format(printf, 1, 2)));
 int wc_fail_hip(const char* where, hipError_t err);
 
 namespace wc {

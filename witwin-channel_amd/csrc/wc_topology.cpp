@@ -1,7 +1,7 @@
 // Host part of scene compilation: the welded edge candidates of a mesh and the
 // convex hulls of its coplanar groups (what the public call does before any
-// kernel runs). Plain C++ on host arrays; no device work.
-#include "wc_api_internal.h"
+// kernel runs). Plain C++ on host arrays; no device work, no HIP.
+#include "wc_error.h"
 #include "../../include/wcmi.h"
 
 #include <algorithm>

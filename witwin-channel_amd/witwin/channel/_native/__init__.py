@@ -18,7 +18,9 @@ from typing import Any
 import torch
 
 _LIB_PATH = Path(__file__).resolve().parent / "libwcmi.so"
+_HOST_LIB_PATH = _LIB_PATH.with_name("libwcmi_host.so")
 _lib: ctypes.CDLL | None = None
+_host_lib: ctypes.CDLL | None = None
 
 c_int = ctypes.c_int
 c_float = ctypes.c_float
@@ -298,6 +300,9 @@ _SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
 }
 
 
+# entry points that libwcmi_host.so holds too: host arrays only
+_HOST_FUNCTIONS = ("wc_edge_candidates", "wc_group_hulls")
+
 # int-returning entry points whose result is a value, not a status
 _VALUE_RETURNING = frozenset({"wc_abi_version", "wc_bvh_node_count", "wc_vjp_partial_stride",
                               "wc_vjp_partial_rows"})
@@ -313,20 +318,41 @@ def load() -> ctypes.CDLL:
     global _lib
     if _lib is not None:
         return _lib
-    path = Path(os.environ.get("WCMI_LIBRARY", str(_LIB_PATH)))
+    _lib = _open(Path(os.environ.get("WCMI_LIBRARY", str(_LIB_PATH))), list(_SIGNATURES))
+    return _lib
+
+
+def load_host() -> ctypes.CDLL:
+    """Load libwcmi_host.so once. Scene compilation calls it so that libwcmi.so
+    is not loaded before the GPU runtime: the libraries which the runtime opens
+    leave the thread's TLS table out of date, every TLS access of the program
+    (each allocation, each launch) then takes the slow way, and libwcmi.so,
+    opened after them, is what brings the table up to date (a held 1-cell
+    forward takes 31 us, 35 in the other order; glibc 2.35). libwcmi.so exports
+    the same functions and stands in where only it is installed."""
+
+    global _host_lib
+    if _host_lib is None:
+        if not _HOST_LIB_PATH.exists():
+            return load()
+        _host_lib = _open(_HOST_LIB_PATH, [*_HOST_FUNCTIONS, "wc_last_error"])
+    return _host_lib
+
+
+def _open(path: Path, names: list[str]) -> ctypes.CDLL:
     if not path.exists():
         raise NativeLibraryError(
-            f"libwcmi.so not found at {path}; build it with "
+            f"{path.name} not found at {path}; build it with "
             "`python witwin-channel_amd/build_native.py` (there is no CPU fallback)"
         )
     lib = ctypes.CDLL(str(path))
-    for name, (restype, argtypes) in _SIGNATURES.items():
+    for name in names:
+        restype, argtypes = _SIGNATURES[name]
         fn = getattr(lib, name, None)
         if fn is None:
-            raise NativeLibraryError(f"libwcmi.so does not export {name}")
+            raise NativeLibraryError(f"{path.name} does not export {name}")
         fn.restype = restype
         fn.argtypes = argtypes
-    _lib = lib
     return lib
 
 
@@ -335,7 +361,15 @@ def exported_symbols() -> list[str]:
 
 
 def call(name: str, *args: Any) -> Any:
-    lib = load()
+    return _checked(load(), name, args)
+
+
+def call_host(name: str, *args: Any) -> Any:
+    """``call`` for the entry points of libwcmi_host.so."""
+    return _checked(load_host(), name, args)
+
+
+def _checked(lib: ctypes.CDLL, name: str, args: tuple) -> Any:
     fn = getattr(lib, name)
     status = fn(*args)
     if fn.restype is c_int and name not in _VALUE_RETURNING and status != 0:

@@ -348,9 +348,9 @@ def build_edge_table(vertices: np.ndarray, faces: np.ndarray, face_group: np.nda
     ids = np.empty((3 * n_faces, 6), np.int64)
     pid = np.empty(3 * n_faces, np.int64)
     count = np.zeros(1, np.int32)
-    _native.call("wc_edge_candidates", q.ctypes.data, int(q.shape[0]), tri.ctypes.data, n_faces, fstruct.ctypes.data,
-                 vbase.ctypes.data, int(vbase.shape[0]), group.ctypes.data, material.ctypes.data, ev.ctypes.data,
-                 ids.ctypes.data, pid.ctypes.data, count.ctypes.data)
+    _native.call_host("wc_edge_candidates", q.ctypes.data, int(q.shape[0]), tri.ctypes.data, n_faces,
+                      fstruct.ctypes.data, vbase.ctypes.data, int(vbase.shape[0]), group.ctypes.data,
+                      material.ctypes.data, ev.ctypes.data, ids.ctypes.data, pid.ctypes.data, count.ctypes.data)
     ev, ids, pid = (x[:int(count[0])] for x in (ev, ids, pid))
     g = edge_geometry(v, ev)
     keep = g["length"] >= 1e-9
@@ -569,9 +569,9 @@ def group_hulls(vertices: np.ndarray, faces: np.ndarray, group_face_offset: np.n
         raise IndexError(f"{g} groups with {first.shape[0]} face offsets")
     offset = np.zeros(g + 1, np.int32)
     points = np.empty((3 * int(members.shape[0]) * 2, 3), np.float64)
-    _native.call("wc_group_hulls", verts.ctypes.data, int(verts.shape[0]), tri.ctypes.data, int(tri.shape[0]),
-                 first.ctypes.data, members.ctypes.data, int(members.shape[0]), plane.ctypes.data, g,
-                 offset.ctypes.data, points.ctypes.data)
+    _native.call_host("wc_group_hulls", verts.ctypes.data, int(verts.shape[0]), tri.ctypes.data, int(tri.shape[0]),
+                      first.ctypes.data, members.ctypes.data, int(members.shape[0]), plane.ctypes.data, g,
+                      offset.ctypes.data, points.ctypes.data)
     return offset, np.ascontiguousarray(points[:int(offset[g])])
 
 
@@ -612,6 +612,7 @@ class DeviceScene:
             raise ValueError(f"bvh must be one of {BVH_BUILDERS}, got {bvh!r}")
         self.device = device
         self.bvh = bvh
+        torch.empty(1, device=device)  # the device's runtime before libwcmi.so (_native.load_host)
         mats = compiled.materials
         f = compiled.face_count
         f32, i32 = np.float32, np.int32

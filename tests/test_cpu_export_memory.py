@@ -55,7 +55,7 @@ def export(monkeypatch):
         monkeypatch.setattr(_native, "call", call)
         monkeypatch.setattr(_native, "stream_handle", lambda device=None: 0)
         monkeypatch.setattr(torch, "empty", short)
-        dscene = SimpleNamespace(device=torch.device("cpu"), view=SimpleNamespace(edge_count=0), edge_count=0,
+        dscene = SimpleNamespace(device=torch.device("cpu"), view=SimpleNamespace(edge_count=0, face_count=770), edge_count=0,
                                  ref=lambda: None)
         inputs = SimpleNamespace(total_cells=1, tile_count=1, tiles=torch.zeros(2, dtype=torch.int32),
                                  view=_native.WcSolve(), pair_cell=torch.zeros(1, dtype=torch.int32))

@@ -82,6 +82,29 @@ def test_masked_export_equals_per_cell_export(device, monkeypatch, tx_count, rx_
             assert torch.equal(a, b), name
 
 
+@pytest.mark.parametrize("rx_count,per_cell", [((1,), True), ((64,), True), ((65,), False)])
+def test_both_exports_either_side_of_few_candidates(device, rx_count, per_cell):
+    """Five chains over ten triangles: per cell up to 64 cells. The rows are the same either way."""
+    from witwin.core import Mesh, PhysicalMaterial, Structure
+
+    def wall(k):
+        x, y = (80.0 * np.cos(k), 80.0 * np.sin(k))
+        v = torch.tensor([[x, y, 0.0], [x - 30.0 * y / 80.0, y + 30.0 * x / 80.0, 0.0],
+                          [x - 30.0 * y / 80.0, y + 30.0 * x / 80.0, 60.0], [x, y, 60.0]])
+        return Structure(Mesh(v, torch.tensor([[0, 1, 2], [0, 2, 3]])), PhysicalMaterial(eps_r=4.0, sigma_e=0.01),
+                         surface_id=k)
+
+    scene = Scene(structures=[wall(k) for k in range(5)], endpoints=[])
+    dscene, inputs = _inputs(device, 1, rx_count, ("los", "reflection", "transmission"), 1, {}, scene)
+    assert inputs.view.max_tx_chains == 5 and dscene.view.face_count == 10
+    assert engine._few_candidates(dscene, inputs) == per_cell
+    masked = engine._export_rows(dscene, inputs, 1, None, [engine.export_masks(dscene, inputs)])
+    plain = engine._export_rows(dscene, inputs, 1, None, [None])
+    for name in ("tx_id", "rx_id", "component_id", "depth", "primitive_sequence"):
+        assert torch.equal(masked[name], plain[name]), name
+    torch.testing.assert_close(masked["path_field"], plain["path_field"], rtol=2e-6, atol=1e-12)
+
+
 def test_masked_export_without_candidates(device, monkeypatch):
     dscene, inputs = _inputs(device, 2, (5, 70), ("los", "reflection"), 1, {}, Scene(structures=[], endpoints=[]))
     masked, plain = _both(monkeypatch, dscene, inputs, 1, None)

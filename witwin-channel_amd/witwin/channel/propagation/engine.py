@@ -656,6 +656,22 @@ def export_masks(dscene: DeviceScene, inputs: SolveInputs) -> torch.Tensor | Non
         return None
 
 
+def _few_candidates(dscene: DeviceScene, inputs: SolveInputs) -> bool:
+    """Whether the per-cell export is the faster one: its two kernels test
+    everything twice in one lane per cell, where the masked one launches three
+    to five more and keeps each row's candidate in memory in between. Times per
+    cell / with masks (ms), 300,000 cells unless stated: line of sight over 2
+    triangles 0.77 / 0.91, over 34 0.77 / 0.83, over 770 0.88 / 0.74; line of
+    sight and transmission over 18 triangles 0.98 / 0.89; one reflection chain
+    1.04 / 1.17, two 1.14 / 1.20, three 1.28 / 1.19; nine chains 1.79 / 1.20,
+    but 0.41 / 0.44 for one cell and 0.46 / 0.47 for 16; four edges
+    1.99 / 1.67."""
+    chains = int(inputs.view.max_tx_chains)
+    if dscene.edge_count and int(inputs.view.components) & 4:
+        return False
+    return int(dscene.view.face_count) <= 16 and chains <= (8 if inputs.total_cells <= 64 else 2)
+
+
 def export_rows(dscene: DeviceScene, inputs: SolveInputs, *, width: int,
                 max_paths_per_pair: int | None = None) -> dict[str, Any]:
     """Explicit path rows in canonical order: pairs rx-major, tx-minor; inside a
@@ -667,7 +683,7 @@ def export_rows(dscene: DeviceScene, inputs: SolveInputs, *, width: int,
     canonical pair) describe the kept rows' segmentation; ``dropped`` counts
     identity winners removed by the cap."""
 
-    held = [export_masks(dscene, inputs)]
+    held = [None if _few_candidates(dscene, inputs) else export_masks(dscene, inputs)]
     if held[0] is not None:
         # the masked export takes more memory than the per-cell one (its masks,
         # and rows below the gain floor): where it does not fit, that one may

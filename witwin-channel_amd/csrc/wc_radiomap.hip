@@ -1750,34 +1750,55 @@ __host__ __device__ inline FanPlane fan_plane(const ShadowFrame& f) {
     return p;
 }
 
-__host__ __device__ inline bool fan_plane_misses(const FanPlane& p, const Tri& tri) {
+// the vertices lie on one side of the plane
+__host__ __device__ inline bool fan_plane_aside(const FanPlane& p, const Tri& tri) {
     const float vx[3] = {tri.v0.x - p.ax, tri.v1.x - p.ax, tri.v2.x - p.ax};
     const float vy[3] = {tri.v0.y - p.ay, tri.v1.y - p.ay, tri.v2.y - p.ay};
     const float vz[3] = {tri.v0.z - p.az, tri.v1.z - p.az, tri.v2.z - p.az};
-    bool above = true, below = true, behind = true, out_a = true, out_b = true;
+    bool above = true, below = true;
     for (int k = 0; k < 3; ++k) {
         const float sd = p.mx * vx[k] + p.my * vy[k] + p.mz * vz[k];
-        const float x = p.dx * vx[k] + p.dy * vy[k] + p.dz * vz[k];
-        const float y = p.wx * vx[k] + p.wy * vy[k] + p.wz * vz[k];
         above = above && sd > p.tol;
         below = below && sd < -p.tol;
+    }
+    return above || below;
+}
+
+// their in-plane coordinates lie beyond one side of (T, A, B)
+__host__ __device__ inline bool fan_plane_outside(const FanPlane& p, const Tri& tri) {
+    const float vx[3] = {tri.v0.x - p.ax, tri.v1.x - p.ax, tri.v2.x - p.ax};
+    const float vy[3] = {tri.v0.y - p.ay, tri.v1.y - p.ay, tri.v2.y - p.ay};
+    const float vz[3] = {tri.v0.z - p.az, tri.v1.z - p.az, tri.v2.z - p.az};
+    bool behind = true, out_a = true, out_b = true;
+    for (int k = 0; k < 3; ++k) {
+        const float x = p.dx * vx[k] + p.dy * vy[k] + p.dz * vz[k];
+        const float y = p.wx * vx[k] + p.wy * vy[k] + p.wz * vz[k];
         behind = behind && y < -p.tol;
         out_a = out_a && p.at_x * x + p.at_y * y > p.tol;
         out_b = out_b && p.bt_x * (x - p.len) + p.bt_y * y > p.tol;
     }
-    return above || below || behind || out_a || out_b;
+    return behind || out_a || out_b;
+}
+
+__host__ __device__ inline bool fan_plane_misses(const FanPlane& p, const Tri& tri) {
+    return fan_plane_aside(p, tri) || fan_plane_outside(p, tri);
 }
 
 // Shadow bins of every (transmitter, edge) over all triangles outside the
 // edge's own face groups (which the leg test ignores): one wavefront per pair,
-// lane l pre-tests triangles l, l + 64, ... The few that reach the edge's fan
-// triangle (3 % on the canyon, so most rounds of 64 have one) queue in LDS and
-// take the double-precision section test 64 at a time; tested where they are
-// met, nearly every round paid for one. 64 transmitters of the canyon (49,408
-// pairs, 770 triangles): 272 us tested at once, 174 us queued.
+// 128 triangles a round, of which lane l pre-tests l and l + 64. VALU bound. The
+// plane test comes first and its sides only where a lane crosses the plane:
+// neighbouring triangles mostly lie on one side of it together. The few that
+// reach the fan triangle (3 % on the canyon, next to none on open terrain)
+// queue in LDS and take the double-precision section test 64 at a time; tested
+// where they are met, a street's rounds nearly all run one. Tested at once /
+// queued: 64 transmitters of the canyon (49,408 pairs, 770 triangles)
+// 276 / 175 us, 3,076 street edges x 8 (3,074 triangles) 296 / 233 us, 25,280
+// pairs on 2,072 terrain triangles 166 / 169 us.
+constexpr int kShadowRound = 2;  // triangles a lane pre-tests per round
 __global__ void __launch_bounds__(256) edge_shadow_kernel(SceneView s, wc_solve q,
                                                           unsigned long long* __restrict__ shadow, long long wave_base) {
-    __shared__ int queue[4][128];
+    __shared__ int queue[4][64 * (kShadowRound + 1)];
     const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const long long pair = wave_base + (long long)blockIdx.x * (blockDim.x >> 6) + wid;
     const int edges = s.edge_count;
@@ -1788,30 +1809,49 @@ __global__ void __launch_bounds__(256) edge_shadow_kernel(SceneView s, wc_solve 
     unsigned long long bits = 0;
     if (f.valid) {
         const FanPlane plane = fan_plane(f);
-        int queued = 0;  // the same in every lane
-        for (int base = 0; base < s.face_count || queued > 0; base += 64) {
-            const int k = base + lane;
-            bool reach = false;
-            if (k < s.face_count) {
-                const Tri tri = s.faces[k];
-                const int group = __float_as_int(tri.v0.w);
-                reach = group != e.group0 && group != e.group1 && !fan_plane_misses(plane, tri);
+        int queued = 0;  // the same in every lane, below 64 when a round starts
+        const Tri* at = s.faces + lane;
+        auto crosses = [&](const Tri& tri) {
+            const int group = __float_as_int(tri.v0.w);
+            return group != e.group0 && group != e.group1 && !fan_plane_aside(plane, tri);
+        };
+        for (int base = 0; base < s.face_count; base += 64 * kShadowRound, at += 64 * kShadowRound) {
+            const bool last = base + 64 * kShadowRound >= s.face_count;
+            bool reach[kShadowRound], any = false;
+            Tri tri[kShadowRound];
+#pragma unroll
+            for (int u = 0; u < kShadowRound; ++u) {
+                const bool in = base + 64 * u + lane < s.face_count;
+                tri[u] = in ? at[64 * u] : s.faces[0];
+                reach[u] = in && crosses(tri[u]);
+                any = any || reach[u];
             }
-            const unsigned long long ball = __ballot(reach);
-            if (reach) queue[wid][queued + (int)__popcll(ball & ((1ull << lane) - 1ull))] = k;
-            queued += (int)__popcll(ball);
-            if (queued < 64 && base + 64 < s.face_count) continue;
+            // neighbouring triangles mostly lie on one side of the plane together
+            if (__ballot(any) != 0ull) {
+                any = false;
+#pragma unroll
+                for (int u = 0; u < kShadowRound; ++u) {
+                    reach[u] = reach[u] && !fan_plane_outside(plane, tri[u]);
+                    any = any || reach[u];
+                }
+            }
+            if (__ballot(any) == 0ull && !(last && queued > 0)) continue;
+#pragma unroll
+            for (int u = 0; u < kShadowRound; ++u) {
+                const unsigned long long ball = __ballot(reach[u]);
+                if (reach[u])
+                    queue[wid][queued + (int)__popcll(ball & ((1ull << lane) - 1ull))] = base + 64 * u + lane;
+                queued += (int)__popcll(ball);
+            }
+            if (queued < 64 && !(last && queued > 0)) continue;
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            const int item = lane < queued ? queue[wid][lane] : -1;
-            const int carry = lane + 64 < queued ? queue[wid][lane + 64] : -1;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if (carry >= 0) queue[wid][lane] = carry;
-            queued = queued > 64 ? queued - 64 : 0;
-            if (item >= 0) bits |= triangle_shadow_bins(f, s.faces[item]);
+            while (queued >= 64 || (last && queued > 0)) {
+                const int n = min(queued, 64);
+                queued -= n;
+                if (lane < n) bits |= triangle_shadow_bins(f, s.faces[queue[wid][queued + lane]]);
+            }
         }
     }
     for (int off = 1; off < 64; off <<= 1) {
@@ -1827,9 +1867,8 @@ __global__ void __launch_bounds__(256) edge_shadow_kernel(SceneView s, wc_solve 
 // pass the pre-test wait in a short list per lane, and the wavefront runs their
 // double-precision section tests together when a list fills: tested where the
 // walk meets them, nearly every step would run one for a lane or two.
-// The kernel above reads every triangle for every edge; it stays for small
-// meshes, where a fan triangle meets a good part of the tree
-// (see edge_shadow_walks).
+// The kernel above reads every triangle for every edge and stays where that is
+// less (edge_shadow_walks).
 constexpr int kShadowList = 12;  // per lane; a step adds at most four
 constexpr int kShadowLanes = 16;
 
@@ -1926,12 +1965,34 @@ __global__ void __launch_bounds__(256) edge_shadow_walk_kernel(SceneView s, wc_s
     if (pair < pairs && part == 0) shadow[pair] = bits;
 }
 
-// Which shadow kernel, by the triangles the other one reads per edge. Measured,
-// walk against all triangles: 772 edges of one transmitter on 770 triangles
-// 0.298 / 0.024 ms, 64 transmitters there 0.597 / 0.174 ms (a street's fan
-// meets much of so small a tree), 8 transmitters of the scaled city (134,850
-// triangles) 1.22 / 5.06 ms.
-__host__ inline bool edge_shadow_walks(int face_count) { return face_count >= 16384; }
+// Which shadow kernel. All triangles cost 2 to 4 ps per (pair, triangle) once
+// they fill the chip and 5 us per 1,000 triangles when they do not; a walk
+// costs 4 to 12 ns per pair, and no less than its longest chain of nodes: 0.1 to
+// 0.2 ms on terrain, 0.4 to 1 ms in streets, whose fans meet much of the tree.
+// Measured, all triangles / walk (ms): terrain of 2,072 triangles, 202,240 pairs
+// 1.18 / 0.86; 8,058: 12,149 pairs 0.25 / 0.16, 97,192 pairs 1.88 / 0.63;
+// 16,320: 24,575 pairs 0.96 / 0.29; 32,378: 40 pairs 0.17 / 0.13, 320 pairs
+// 0.17 / 0.23, 2,560 pairs 0.25 / 0.23; streets of 770 triangles, 49,408 pairs
+// 0.18 / 0.61; 3,074: 196,864 pairs 1.69 / 2.59; 6,146: 49,184 pairs 0.82 /
+// 1.28, 393,472 pairs 5.85 / 5.36; 12,290: 12,292 pairs 0.45 / 0.98, 98,336
+// pairs 2.97 / 2.17; eight transmitters of the scaled city (134,850) 5.06 / 1.22. From 4e8 tests on the walk loses on neither kind of
+// scene; with few pairs it wins where a wavefront's 0.25 ms over 49,152
+// triangles is more than any of its chains.
+__host__ inline bool edge_shadow_walks(long long pairs, int face_count) {
+    return face_count >= 49152 || (face_count >= 4096 && pairs * face_count >= 400000000LL);
+}
+
+// Whether the table pays for itself: up to 4e9 tests it is a few milliseconds
+// at most, and beyond them a pair's walk (5 ns) has to be worth it to that
+// transmitter's receivers. With / without the table, 64 transmitters: 8,058
+// triangles and 1 receiver each 7.7 / 4.0 ms, 16 receivers 11.7 / 8.4, 1,024
+// receivers 158 / 171; 32,378 triangles and 256 receivers 652 / 645. The
+// visibility test alone is exact.
+constexpr long long kShadowBudget = 4000000000LL;
+constexpr int kShadowCells = 512;
+__host__ inline bool edge_shadow_pays(const wc_solve& q, long long pairs, int face_count) {
+    return pairs * face_count <= kShadowBudget || q.total_cells / q.tx_count >= kShadowCells;
+}
 
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WC_VIS_WAVES_PER_EU)))
 diff_visibility_kernel(SceneView s, wc_solve q, unsigned* __restrict__ masks, int words, long long waves,
@@ -2583,11 +2644,6 @@ static int device_cus() {
     return cached_cus;
 }
 
-// The brute-force shadow table costs transmitters x edges x triangles
-// segment-plane tests; above this many it is skipped (the visibility test
-// alone is exact).
-constexpr long long kShadowBudget = 4000000000LL;
-
 static void launch_diff_visibility(const SceneView& s, const wc_solve& q, const wc_radiomap_out& o, hipStream_t st) {
     const int words = mask_words(s.edge_count);
     if (words == 0) return;
@@ -2595,8 +2651,8 @@ static void launch_diff_visibility(const SceneView& s, const wc_solve& q, const 
                                                   partial_bytes(q.total_cells, q.lanes_per_cell));
     unsigned long long* shadow = nullptr;
     const long long pairs = (long long)q.tx_count * s.edge_count;
-    const bool walk = edge_shadow_walks(s.face_count);
-    if (pairs > 0 && (walk || pairs * (long long)s.face_count <= kShadowBudget)) {
+    const bool walk = edge_shadow_walks(pairs, s.face_count);
+    if (pairs > 0 && edge_shadow_pays(q, pairs, s.face_count)) {
         shadow = reinterpret_cast<unsigned long long*>(
             static_cast<char*>(o.workspace) + shadow_offset(q.total_cells, q.lanes_per_cell, s.edge_count,
                                                             q.max_tx_chains, q.tx_count));

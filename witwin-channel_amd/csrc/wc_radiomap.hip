@@ -1255,11 +1255,19 @@ __device__ __forceinline__ unsigned cull_segment(const SceneView& s, const wc_so
 // Segments of 64 / 16 / 4 / 1 words: heightfield (1,024 tiles, 722 words)
 // 1.90 / 1.50 / 1.13 / 1.18 ms, eight transmitters of the scaled city (12 k
 // tiles, 1.5 k words) 14.1 / 14.6 / 18.0 / 26.4 ms a pass. The shortest
-// segment (4 to 64) that keeps the launch below 200,000 wavefronts.
-constexpr long long kSegWaves = 200000;
+// segment (4 to 64) whose launch stays below a number of wavefronts: how much
+// their fixed costs weigh depends on how unevenly the chains lie. Forward of
+// reflection maps (ms), every segment 64 words and one chunk culled at a time /
+// below 100,000 / below 200,000 wavefronts: up to 2,048 tiles the higher limit,
+// heightfield 1.59 / 1.34 / 1.25, terrain of 8,058 triangles (248 words) 0.83 /
+// 0.77 / 0.72, scaled city (2,048 tiles, 1,227 words) 7.0 / 5.6 / 4.9; beyond,
+// the lower one, terrain (4,096 tiles, 255 words) 1.20 / 1.19 / 1.39, 16
+// transmitters there 2.18 / 2.07 / 2.28, scaled city (4,096 tiles, 104 words)
+// 2.30 / 1.27 / 1.00, (835 words) 6.15 / 5.80 / 4.87.
 __host__ inline int segment_words(long long tile_count, int words) {
+    const long long waves = tile_count <= 2048 ? 200000 : 100000;
     int n = 4;
-    while (n < 64 && tile_count * ((words + n - 1) / n) > kSegWaves) n <<= 1;
+    while (n < 64 && tile_count * ((words + n - 1) / n) > waves) n <<= 1;
     return n;
 }
 

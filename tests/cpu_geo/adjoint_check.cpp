@@ -7,12 +7,13 @@
 // the 2-norm of the difference over the 2-norm of the tangent contraction over
 // the ordinary rows and over the degenerate ones, and the number of non-zeros
 // in masked rows. Then the stored-path sweeps of the radiomap adjoint
-// (wc_path_adjoint.h) against the dual-number evaluators (wc_tangent.h) over
+// (wc_path_adjoint.h) against the dual-number evaluators (plane_tangents.h) over
 // random planes and layered walls: "planes" and "wall_normals", coherent and
 // incoherent.
 #include "hip/hip_runtime.h"
 #include "../../witwin-channel_amd/csrc/wc_rows.hip"
 #include "../../witwin-channel_amd/csrc/wc_path_adjoint.h"
+#include "plane_tangents.h"
 
 #include <cstdio>
 #include <random>

@@ -982,11 +982,10 @@ extern "C" int wc_radiomap_vjp_geometry(const wc_scene* scene, const wc_solve* s
     if (!scene || !solve) return wc_fail("wc_radiomap_vjp_geometry: null argument");
     if (scene->group_count > 0 && !grad_group_plane)
         return wc_fail("wc_radiomap_vjp_geometry: grad_group_plane is required");
-    // There is no edge part: its kernel
-    // stopped with a GPU memory aperture violation whose cause is not
-    // identified (the same device code runs clean under AddressSanitizer in a
-    // CPU build over every edge/receiver pair of that scene). Solves with
-    // diffraction are refused rather than returning a partial gradient.
+    // There is no edge part: an earlier kernel for it, no longer in the tree,
+    // stopped with a GPU memory aperture violation whose cause was not
+    // identified. Solves with diffraction are refused rather than returning a
+    // partial gradient.
     if (scene->edge_count > 0 && (solve->components & kCompDiff))
         return wc_fail("wc_radiomap_vjp_geometry: vertex gradients of diffraction paths are not available; "
                        "solve without diffraction");

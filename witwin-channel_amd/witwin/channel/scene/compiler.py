@@ -86,7 +86,7 @@ class CompiledScene:
     edge_policy: str = "all"
     # [E, 4] int32 vertex ids (a, b, c0, c1) of every edge record (see edge_geometry)
     edge_vertices: np.ndarray = field(default_factory=lambda: np.zeros((0, 4), np.int32))
-    # [E] int32 public id of every edge record: the id path rows report (record_ids)
+    # [E] int32 public id of every edge record: the id path rows report (build_edge_table)
     edge_public_id: np.ndarray = field(default_factory=lambda: np.zeros(0, np.int32))
     # [F] structure of every face and [S] first vertex row of every structure
     face_structure: np.ndarray = field(default_factory=lambda: np.zeros(0, np.int64))

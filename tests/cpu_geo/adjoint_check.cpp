@@ -9,7 +9,7 @@
 // in masked rows. Then the stored-path sweeps of the radiomap adjoint
 // (wc_path_adjoint.h) against the dual-number evaluators (plane_tangents.h) over
 // random planes and layered walls: "planes" and "wall_normals", coherent and
-// incoherent.
+// incoherent, and how far each of the two is from 64 bits.
 #include "hip/hip_runtime.h"
 #include "../../witwin-channel_amd/csrc/wc_rows.hip"
 #include "../../witwin-channel_amd/csrc/wc_path_adjoint.h"
@@ -148,6 +148,24 @@ static void contract_dual(const C3<Dual<N>>& f, const V3<Dual<N>>& dir, const V3
     for (int i = 0; i < N; ++i) d[i] = (double)g.re * c.re.d[i] + (double)g.im * c.im.d[i];
 }
 
+// the same slot by central differences of the double evaluation, at steps of
+// 1e-6 (metres, or parts of a normal: up to 1e-4 rad of phase, so 1e-8 of the
+// derivative are lost to curvature and 1e-8 to rounding)
+template <class Path>
+static double contract_double(Path&& path, const PathCotangent& w, const V3<float>& rx_pol) {
+    auto coefficient = [&](double step) {
+        V3<double> dir;
+        const C3<double> f = path(step, dir);
+        return project_receiver(f, dir, lift3<double>(rx_pol));
+    };
+    const double h = 1.0e-6;
+    const Cx<double> a = coefficient(-h), b = coefficient(h), c = coefficient(0.0);
+    const double re = (b.re - a.re) / (2.0 * h), im = (b.im - a.im) / (2.0 * h), sp = w.sp;
+    const Cx<double> g = w.coherent ? Cx<double>{w.a.re * sp, w.a.im * sp}
+                                    : Cx<double>{c.re * w.inc * sp * sp, c.im * w.inc * sp * sp};
+    return g.re * re + g.im * im;
+}
+
 static void check_paths(int n, double freq, bool coherent) {
     std::mt19937 gen(coherent ? 7 : 8);
     std::uniform_real_distribution<float> u01(0.0f, 1.0f);
@@ -186,7 +204,8 @@ static void check_paths(int n, double freq, bool coherent) {
     const double k_d = freq * kTwoPi / kC0;
     const float f = (float)freq;
     constexpr int DM = kMaxDepth;
-    Sum planes, wall_n;
+    Sum planes, wall_n;             // sweep against the dual numbers
+    Sum planes64[2], wall_n64[2];  // sweep and dual numbers against 64 bits
     for (int i = 0; i < n; ++i) {
         PathCotangent w;
         w.coherent = coherent;
@@ -220,7 +239,25 @@ static void check_paths(int n, double freq, bool coherent) {
         PlaneGrad<DM> bp, bn;
         reflection_planes<DM>(s, depth, groups, mats, tx, rx, txp, rxp, f, k_d, length, w, bp);
         const int nw = i % (DM + 1);
-        straight_normals<DM>(s, nw, hits, tx, rx, txp, rxp, f, k_d, dist, w, bn);
+        // carrier length in double, as the forward pass has it
+        double carrier = dist;
+        for (int b = 0; b < nw; ++b) {
+            double o;
+            const double ct = std::fabs(dot((to_d(rx) - to_d(tx)) * (1.0 / dist), group_normal(s, groups[b], o)));
+            for (int l = 0; l < lc[mats[b]]; ++l) carrier -= (double)lt[lo[mats[b]] + l] * std::max(ct, 1e-6);
+        }
+        straight_normals<DM>(s, nw, hits, tx, rx, txp, rxp, f, k_d, carrier, w, bn);
+        // the planes in double, the one of `slot` moved by `step`
+        auto move_plane = [&](int slot, double step, V3<double>* nd, double* od) {
+            for (int b = 0; b < DM; ++b) {
+                double o;
+                nd[b] = to_d(to_f(group_normal(s, groups[b], o)));
+                od[b] = (double)(float)o;
+                if (slot / 4 != b) continue;
+                double* part[4] = {&nd[b].x, &nd[b].y, &nd[b].z, &od[b]};
+                *part[slot % 4] += step;
+            }
+        };
         for (int slot = 0; slot < 4 * DM; ++slot) {
             V3<D1> nv[DM];
             D1 off[DM];
@@ -240,16 +277,37 @@ static void check_paths(int n, double freq, bool coherent) {
                 contract_dual<1>(reflection_tangent_planes(s, depth, groups, nv, off, tx, rx, txp, f, k_d, length, dir),
                                  dir, rxp, w, d);
                 planes.add(value(bp), d[0]);
+                const double want = contract_double(
+                    [&](double step, V3<double>& dir64) {
+                        V3<double> nd[DM];
+                        double od[DM];
+                        move_plane(slot, step, nd, od);
+                        return reflection_tangent_planes(s, depth, groups, nd, od, tx, rx, txp, f, k_d, 0.0, dir64);
+                    },
+                    w, rxp);
+                planes64[0].add(value(bp), want);
+                planes64[1].add(d[0], want);
             }
             if (b < nw && c < 3) {
-                contract_dual<1>(transmission_tangent_walls(s, nw, hits, nv, tx, rx, txp, f, k_d, dist, dir), dir, rxp,
+                contract_dual<1>(transmission_tangent_walls(s, nw, hits, nv, tx, rx, txp, f, k_d, carrier, dir), dir, rxp,
                                  w, d);
                 wall_n.add(value(bn), d[0]);
+                const double want = contract_double(
+                    [&](double step, V3<double>& dir64) {
+                        V3<double> nd[DM];
+                        double od[DM];
+                        move_plane(slot, step, nd, od);
+                        return transmission_tangent_walls(s, nw, hits, nd, tx, rx, txp, f, k_d, 0.0, dir64);
+                    },
+                    w, rxp);
+                wall_n64[0].add(value(bn), want);
+                wall_n64[1].add(d[0], want);
             }
         }
     }
     const char* mode = coherent ? "coherent" : "incoherent";
-    std::printf("%s planes %.3e\n%s wall_normals %.3e\n", mode, planes.error(), mode, wall_n.error());
+    std::printf("%s planes %.3e %.3e %.3e\n%s wall_normals %.3e %.3e %.3e\n", mode, planes.error(), planes64[0].error(),
+                planes64[1].error(), mode, wall_n.error(), wall_n64[0].error(), wall_n64[1].error());
 }
 
 int main() {

@@ -1,12 +1,17 @@
 // Stored paths whose reflecting planes (n, c) or wall normals carry the
-// derivatives, as the adjoint check evaluates them with dual numbers in the
-// rounding steps of the kernels' own tangents (wc_tangent.h). Endpoints,
-// frequency and materials are constants.
+// derivatives, as the adjoint checks evaluate them: with dual numbers in the
+// rounding steps of the kernels' own tangents (wc_tangent.h), or in double.
+// Endpoints, frequency and materials are constants.
 #pragma once
 
 #include "../../witwin-channel_amd/csrc/wc_tangent.h"
 
 namespace wc {
+
+// in double the phase follows the length itself
+template <> struct PhaseOf<double> {
+    static double make(double, double L, double k_d, double) { return -(k_d * L); }
+};
 
 template <typename R>
 __device__ inline C3<R> reflection_tangent_planes(const SceneView& s, int depth, const int* faces, const V3<R>* nrm,

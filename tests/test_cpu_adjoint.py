@@ -52,3 +52,15 @@ def test_stored_path_sweeps_equal_tangents(report, mode):
     # a path's own field weighs the incoherent cotangent: one more rounded factor of its size
     for kind in ("planes", "wall_normals"):
         assert rows[kind][0] < 5.0e-5, kind
+
+
+@pytest.mark.parametrize("mode", ["coherent", "incoherent"])
+@pytest.mark.parametrize("kind", ["planes", "wall_normals"])
+def test_stored_path_sweeps_are_no_farther_from_64_bits(report, mode, kind):
+    """Against central differences in double. Both float32 sides carry the same
+    rounded values (the interior phases move a derivative by 3e-5; an incoherent
+    sum keeps only the amplitude's derivative, whose planes lose 1e-3 of it) and
+    differ in the derivatives' own roundings: a quarter is the room for those."""
+    sweep, duals = next([float(x) for x in r[3:]] for r in report if r[:2] == [mode, kind])
+    assert sweep < 1.25 * duals
+    assert duals < (2.0e-3 if (mode, kind) == ("incoherent", "planes") else 6.0e-5)

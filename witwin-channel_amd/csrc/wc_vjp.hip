@@ -402,7 +402,8 @@ template <int DM> struct LanePlanes {
 // Line-of-sight paths have no geometry (depth 0). Bound by the atomics: on the
 // heightfield (32,738 triangles, 125 k paths of depth 2) 696 us with dual
 // tangents and one atomic per lane, 547 us with the sweep, 148 us with the
-// groups' lanes summed first (flush_planes).
+// groups' lanes summed first (flush_planes). Error against 64 bits as the dual
+// numbers': 2.9e-5 for coherent planes, 3.2e-5 for wall normals.
 template <int DM>
 __device__ __forceinline__ void geometry_path(const SceneView& s, const wc_solve& q, const wc_adjoint& ga, int t,
                                               int cell, int desc, LanePlanes<DM>& out) {

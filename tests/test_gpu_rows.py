@@ -647,3 +647,34 @@ def test_path_los_export_matches_closed_form(device):
     err = np.abs(out["path_gain"].cpu().numpy().astype(np.float64) - gain)
     assert np.all(err <= 2e-5 * gain + 1e-6 * whole), float((err / (gain + whole)).max())
     np.testing.assert_array_equal(out["path_gain_matrix"].cpu().numpy()[ti, ri], out["path_gain"].cpu().numpy())
+
+
+@pytest.mark.parametrize("op", ["free_space", "layer_stack"])
+@pytest.mark.parametrize("rows", [8191, 8192, 8193, 12289])
+def test_frequency_gradient_sums_every_row(device, op, rows):
+    """The frequency gradient of many rows (one workgroup up to 8,191, chunks of
+    4,096 from there, the last with the remainder; behind the layer sums in the
+    workspace for layer stacks) is the sum of its slices'. Rows' partials are the
+    same bits in both and add in float64, so only the float32 results round: half
+    an ulp of the total and of every slice."""
+    rng = np.random.default_rng(rows)
+    t = lambda a: torch.as_tensor(np.asarray(a, np.float32)).to(device)  # noqa: E731
+    if op == "free_space":
+        args = [t(rng.uniform(0, 100, (rows, 3))), t(rng.uniform(0, 100, (rows, 3))), t(rng.uniform(0.1, 2, rows)),
+                t(rng.normal(size=(rows, 3))), t(rng.normal(size=(rows, 3)))]
+        gain = t(rng.uniform(-1, 1, rows))
+        grad = lambda s: F.field_free_space_backward(*(a[s].contiguous() for a in args), frequency_hz=3.5e9,  # noqa: E731
+                                                     grad_path_gain=gain[s].contiguous())["grad_frequency"]
+    else:
+        csr = _csr([[(0.1, 4.0, 0.01, 1.0)], [(0.05, 2.5, 0.0, 1.0), (0.02, 6.0, 0.03, 1.0)]], device)
+        cos = t(rng.uniform(0.1, 1.0, rows))
+        mid = torch.as_tensor(rng.integers(0, 2, rows).astype(np.int32)).to(device)
+        grads = [t(rng.uniform(-1, 1, rows)) for _ in M.EM_LAYER_STACK_FIELDS]
+        grad = lambda s: M.em_layer_stack_backward(  # noqa: E731
+            cos[s].contiguous(), mid[s].contiguous(), **csr, grad_outputs=[g[s].contiguous() for g in grads],
+            frequency_hz=3.5e9, need_cos_theta=False, need_layers=True, need_frequency=True)["grad_frequency"]
+    _say(f"case: {op}, {rows} rows")
+    got = float(grad(slice(0, rows)))
+    slices = [float(grad(slice(k, min(k + 1000, rows)))) for k in range(0, rows, 1000)]
+    assert abs(got) > 0.0
+    assert abs(got - math.fsum(slices)) <= 2.0 ** -24 * (abs(got) + math.fsum(abs(s) for s in slices))

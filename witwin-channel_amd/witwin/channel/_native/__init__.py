@@ -329,9 +329,12 @@ def load_host() -> ctypes.CDLL:
     (each allocation, each launch) then takes the slow way, and libwcmi.so,
     opened after them, is what brings the table up to date (a held 1-cell
     forward takes 31 us, 35 in the other order; glibc 2.35). libwcmi.so exports
-    the same functions and stands in where only it is installed."""
+    the same functions: once loaded it serves them too, as any library opened
+    after it would bring the table out of date again."""
 
     global _host_lib
+    if _lib is not None:
+        return _lib
     if _host_lib is None:
         if not _HOST_LIB_PATH.exists():
             return load()

@@ -92,15 +92,19 @@ def kernel_time(fn, stream, reps: int = 5, before=None) -> float:
     return sum(a.elapsed_time(b) for a, b in zip(starts, ends)) / reps
 
 
-def traffic_bytes(kernel: str, workload: str):
+def traffic_bytes(kernel: str, workload: str, batches: int | None = None):
     """Measured HBM bytes per launch of ``kernel`` on ``workload`` from the
     committed PMC summary (profiles/hbm_traffic.json: FETCH_SIZE + WRITE_SIZE
-    scaled by a copy kernel), or None when no summary matches."""
+    scaled by a copy kernel), or None when no summary matches. A summary taken in
+    another number of ``batches`` is scaled to this one (the same bytes a step)."""
     path = ROOT / "profiles" / "hbm_traffic.json"
     if not path.exists():
         return None
     entry = json.loads(path.read_text()).get("workloads", {}).get(workload, {}).get("kernels", {}).get(kernel)
-    return entry.get("bytes_per_launch") if entry else None
+    if not entry:
+        return None
+    scale = entry["batches"] / batches if batches and "batches" in entry else 1.0
+    return entry["bytes_per_launch"] * scale
 
 
 def descriptor_split(out) -> tuple[int, int]:
@@ -654,7 +658,7 @@ def main() -> int:
         },
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
-                     "traffic": traffic_bytes("chain_validity_pass", workload_name),
+                     "traffic": traffic_bytes("chain_validity_pass", workload_name, city["batches"]),
                      "kernel": "chain_visibility_seg_kernel (with its pass's super_box, super_cull and fill_zero "
                                "launches; average over the batches)",
                      "kernel_ms": city["dom_ms"], "algorithmic_bytes_per_launch": city["dom_bytes"]},

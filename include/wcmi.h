@@ -439,7 +439,8 @@ int wc_paths_emit(const wc_scene* scene, const wc_solve* solve, const int* row_o
  * does not find again, with path_length_m NaN, which the canonical compaction
  * drops. row_list: scratch of total + 2 ints,
  * total = the sum of path_count. Rows kept by the compaction are those of
- * wc_paths_count / wc_paths_emit, in the same order. */
+ * wc_paths_count / wc_paths_emit, in the same order (their numbers may differ
+ * by a rounding: other kernels, other contractions). */
 size_t wc_paths_masks_workspace_bytes(int cells, int lanes_per_cell, int edge_count, int max_tx_chains, int tx_count);
 int wc_paths_count_masked(const wc_scene* scene, const wc_solve* solve, void* workspace, const int* tiles,
                           int tile_count, int* path_count, void* stream);

@@ -99,6 +99,22 @@ def test_cfr_grid_infinite_amplitude(device):
     assert bool(torch.isinf(grid.real).all())
 
 
+def test_cfr_grid_largest_amplitude(device):
+    """A finite amplitude whose product with a row's phasor overflows (3e38 in
+    both parts, an eighth of a turn): the responses that fit float32 are finite."""
+    tau = 2.0 ** -20
+    freqs = (26702.0 + 0.125) / tau + (0.875 / 16.0 / tau) * np.arange(64)
+    a = torch.tensor([[[complex(3.0e38, 3.0e38)]]], dtype=torch.complex64, device=device)
+    got = path.paths_cfr(a, torch.tensor([[tau]], device=device), torch.ones((1, 1), dtype=torch.bool, device=device),
+                         torch.as_tensor(freqs), normalize_delays=False).cpu().numpy().reshape(-1)
+    want = complex(a.cpu().numpy().reshape(-1)[0]) * np.exp(-2.0j * np.pi * ((freqs * tau) % 1.0))
+    fits = np.maximum(np.abs(want.real), np.abs(want.imag)) < 3.3e38
+    assert fits.sum() > 4 and fits[16]
+    for part in ("real", "imag"):  # the magnitude itself is past float32
+        error = getattr(got, part).astype(np.float64)[fits] - getattr(want, part)[fits]
+        assert np.abs(error).max() < 1e-6 * 4.3e38, part
+
+
 def test_cfr_kernel_empty_inputs(device):
     out = path.paths_cfr(torch.zeros((4, 0, 1), dtype=torch.complex64, device=device),
                          torch.zeros((4, 0), device=device), torch.zeros((4, 0), dtype=torch.bool, device=device),

@@ -173,8 +173,9 @@ cfr_grid_kernel(const float* __restrict__ a, const float* __restrict__ tau,
             const int l = __ffsll(left) - 1;
             left &= left - 1;
             const float t = __shfl(my_t, l), ar = __shfl(my_re, l), ai = __shfl(my_im, l);
-            if (!isfinite(ar) || !isfinite(ai)) {
-                // a product of phasors would turn one infinite part into NaN in both
+            if (!isfinite(fabsf(ar) + fabsf(ai))) {
+                // a product of phasors would turn one infinite part into NaN in both, as it
+                // would a finite amplitude whose row factor overflows
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int k = k0 + 32 * (8 * (r >> 2) + 4 * (upper ? 1 : 0) + (r & 3)) + half;

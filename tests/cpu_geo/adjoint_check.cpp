@@ -6,14 +6,12 @@
 // over values that are not numbers. Prints "depth kind errors" per input kind:
 // the 2-norm of the difference over the 2-norm of the tangent contraction over
 // the ordinary rows and over the degenerate ones, and the number of non-zeros
-// in masked rows. Then the stored-path sweeps of the radiomap adjoint
-// (wc_path_adjoint.h) against the dual-number evaluators (plane_tangents.h) over
-// random planes and layered walls: "planes" and "wall_normals", coherent and
-// incoherent, and how far each of the two is from 64 bits.
+// in masked rows. Then the vertex adjoint's path tangents (wc_tangent.h) against
+// the same evaluators in double over random planes and layered walls: "planes"
+// and "wall_normals", coherent and incoherent.
 #include "hip/hip_runtime.h"
 #include "../../witwin-channel_amd/csrc/wc_rows.hip"
-#include "../../witwin-channel_amd/csrc/wc_path_adjoint.h"
-#include "plane_tangents.h"
+#include "../../witwin-channel_amd/csrc/wc_tangent.h"
 
 #include <cstdio>
 #include <random>
@@ -21,6 +19,13 @@
 
 int wc_fail(const char*, ...) { return 1; }
 int wc_fail_hip(const char*, hipError_t) { return 1; }
+
+namespace wc {
+// in double the phase follows the length itself
+template <> struct PhaseOf<double> {
+    static double make(double, double L, double k_d, double) { return -(k_d * L); }
+};
+}  // namespace wc
 
 using namespace wc;
 
@@ -139,12 +144,21 @@ struct Sum {
     double error() const { return std::sqrt(num / den); }
 };
 
+// Cotangent of one path's projected coefficient. Coherent sums fix it per
+// (cell, slot); incoherent ones weight the path's own field.
+struct PathCotangent {
+    Cx<float> a;     // coherent: of the path field
+    float inc;       // incoherent: 2 dL/dgain plus the root-power share
+    bool coherent;
+    float sp;        // sqrt of the transmit power
+};
+
 // <cotangent, d path / d slot i> of a dual evaluation
 template <int N>
 static void contract_dual(const C3<Dual<N>>& f, const V3<Dual<N>>& dir, const V3<float>& rx_pol, const PathCotangent& w,
                           double d[N]) {
     const Cx<Dual<N>> c = project_receiver(f, dir, lift3<Dual<N>>(rx_pol));
-    const Cx<float> g = coefficient_cotangent(w, cval(c));
+    const Cx<float> g = w.coherent ? scale(w.a, w.sp) : scale(cval(c), w.inc * w.sp * w.sp);
     for (int i = 0; i < N; ++i) d[i] = (double)g.re * c.re.d[i] + (double)g.im * c.im.d[i];
 }
 
@@ -204,8 +218,7 @@ static void check_paths(int n, double freq, bool coherent) {
     const double k_d = freq * kTwoPi / kC0;
     const float f = (float)freq;
     constexpr int DM = kMaxDepth;
-    Sum planes, wall_n;             // sweep against the dual numbers
-    Sum planes64[2], wall_n64[2];  // sweep and dual numbers against 64 bits
+    Sum planes, wall_n;
     for (int i = 0; i < n; ++i) {
         PathCotangent w;
         w.coherent = coherent;
@@ -236,8 +249,6 @@ static void check_paths(int n, double freq, bool coherent) {
             r.d[0] = on ? 1.0f : 0.0f;
             return r;
         };
-        PlaneGrad<DM> bp, bn;
-        reflection_planes<DM>(s, depth, groups, mats, tx, rx, txp, rxp, f, k_d, length, w, bp);
         const int nw = i % (DM + 1);
         // carrier length in double, as the forward pass has it
         double carrier = dist;
@@ -246,7 +257,6 @@ static void check_paths(int n, double freq, bool coherent) {
             const double ct = std::fabs(dot((to_d(rx) - to_d(tx)) * (1.0 / dist), group_normal(s, groups[b], o)));
             for (int l = 0; l < lc[mats[b]]; ++l) carrier -= (double)lt[lo[mats[b]] + l] * std::max(ct, 1e-6);
         }
-        straight_normals<DM>(s, nw, hits, tx, rx, txp, rxp, f, k_d, carrier, w, bn);
         // the planes in double, the one of `slot` moved by `step`
         auto move_plane = [&](int slot, double step, V3<double>* nd, double* od) {
             for (int b = 0; b < DM; ++b) {
@@ -268,15 +278,11 @@ static void check_paths(int n, double freq, bool coherent) {
                 off[b] = sd((float)o, slot == 4 * b + 3);
             }
             const int b = slot / 4, c = slot % 4;
-            auto value = [&](const PlaneGrad<DM>& o) {
-                return c == 0 ? o.nrm[b].x : c == 1 ? o.nrm[b].y : c == 2 ? o.nrm[b].z : o.off[b];
-            };
             V3<D1> dir;
             double d[1];
             if (b < depth) {
                 contract_dual<1>(reflection_tangent_planes(s, depth, groups, nv, off, tx, rx, txp, f, k_d, length, dir),
                                  dir, rxp, w, d);
-                planes.add(value(bp), d[0]);
                 const double want = contract_double(
                     [&](double step, V3<double>& dir64) {
                         V3<double> nd[DM];
@@ -285,13 +291,11 @@ static void check_paths(int n, double freq, bool coherent) {
                         return reflection_tangent_planes(s, depth, groups, nd, od, tx, rx, txp, f, k_d, 0.0, dir64);
                     },
                     w, rxp);
-                planes64[0].add(value(bp), want);
-                planes64[1].add(d[0], want);
+                planes.add(d[0], want);
             }
             if (b < nw && c < 3) {
                 contract_dual<1>(transmission_tangent_walls(s, nw, hits, nv, tx, rx, txp, f, k_d, carrier, dir), dir, rxp,
                                  w, d);
-                wall_n.add(value(bn), d[0]);
                 const double want = contract_double(
                     [&](double step, V3<double>& dir64) {
                         V3<double> nd[DM];
@@ -300,14 +304,12 @@ static void check_paths(int n, double freq, bool coherent) {
                         return transmission_tangent_walls(s, nw, hits, nd, tx, rx, txp, f, k_d, 0.0, dir64);
                     },
                     w, rxp);
-                wall_n64[0].add(value(bn), want);
-                wall_n64[1].add(d[0], want);
+                wall_n.add(d[0], want);
             }
         }
     }
     const char* mode = coherent ? "coherent" : "incoherent";
-    std::printf("%s planes %.3e %.3e %.3e\n%s wall_normals %.3e %.3e %.3e\n", mode, planes.error(), planes64[0].error(),
-                planes64[1].error(), mode, wall_n.error(), wall_n64[0].error(), wall_n64[1].error());
+    std::printf("%s planes %.3e\n%s wall_normals %.3e\n", mode, planes.error(), mode, wall_n.error());
 }
 
 int main() {

@@ -1,8 +1,7 @@
-// Reverse-mode (adjoint) forms of the transport operators of wc_em.h and of
-// the stored-path evaluators of wc_tangent.h. One reverse sweep gives every
-// derivative of one path at about the cost of two or three evaluations, where
-// forward mode repeats each operation for every parameter and keeps every
-// intermediate that many times over.
+// Reverse-mode (adjoint) forms of the transport operators of wc_em.h. One
+// reverse sweep gives every derivative of one path at about the cost of two or
+// three evaluations, where forward mode repeats each operation for every
+// parameter and keeps every intermediate that many times over.
 //
 // Conventions: a real loss l; the cotangent of a real x is dl/dx, of a complex
 // z the number g with dl = Re(conj(g) dz), so for holomorphic w = f(z)
@@ -15,39 +14,6 @@
 #include "wc_em.h"
 
 namespace wc {
-
-// Values with the dual numbers' rounding steps (a quotient is a product with
-// the rounded reciprocal) and no tangents. The slab's interior phase reaches
-// hundreds of radians, so one step's rounding of its scale, the same for every
-// path of a material, moves a material's whole gradient by 1e-4: a sweep that
-// stands beside forward-mode derivatives of the same paths (kDualSteps)
-// evaluates where they do. The row operators divide (error of their gradients
-// against 64 bits 4.2e-5, 6.1e-5 with the dual steps).
-using Q = Dual<0>;
-WC_HD Q lq(float v) { return lift<Q>(v); }
-WC_HD V3<Q> lq(const V3<float>& v) { return {lq(v.x), lq(v.y), lq(v.z)}; }
-WC_HD Cx<Q> lq(const Cx<float>& c) { return {lq(c.re), lq(c.im)}; }
-WC_HD C3<Q> lq(const C3<float>& f) { return {lq(f.x), lq(f.y), lq(f.z)}; }
-WC_HD V3<float> vq(const V3<Q>& v) { return {v.x.v, v.y.v, v.z.v}; }
-WC_HD Cx<float> vq(const Cx<Q>& c) { return {c.re.v, c.im.v}; }
-WC_HD C3<float> vq(const C3<Q>& f) { return {vq(f.x), vq(f.y), vq(f.z)}; }
-
-WC_HD void slab_value(float cos_theta, float eps_r, float sigma_e, float mu_r, float gain, float thickness,
-                      float frequency_hz, Cx<float>& r_te, Cx<float>& r_tm) {
-    Cx<Q> te, tm;
-    slab_fresnel(lq(cos_theta), lq(eps_r), lq(sigma_e), lq(mu_r), lq(gain), lq(thickness), lq(frequency_hz), te, tm);
-    r_te = vq(te);
-    r_tm = vq(tm);
-}
-WC_HD C3<float> reflect_value(const C3<float>& value, const V3<float>& incident, const V3<float>& normal, float eps_r,
-                              float sigma_e, float mu_r, float gain, float thickness, float frequency_hz,
-                              V3<float>& outgoing) {
-    V3<Q> out;
-    const C3<Q> v = reflect_c3(lq(value), lq(incident), lq(normal), lq(eps_r), lq(sigma_e), lq(mu_r), lq(gain),
-                               lq(thickness), lq(frequency_hz), out);
-    outgoing = vq(out);
-    return vq(v);
-}
 
 template <typename R> WC_HD Cx<R> conj(const Cx<R>& a) { return {a.re, -a.im}; }
 WC_HD Cx<float> cmulj(const Cx<float>& a, const Cx<float>& g) {  // conj(a) * g
@@ -146,13 +112,11 @@ WC_HD void perp_axis_adj(const V3<float>& a, const V3<float>& b, const V3<float>
 struct SlabGrad {
     float ct, eps, sig, gain, thick, freq;
 };
-template <bool kDualSteps>
 WC_HD void slab_fresnel_adj(float cos_theta, float eps_r, float sigma_e, float mu_r, float gain, float thickness,
                             float frequency_hz, const Cx<float>& g_te, const Cx<float>& g_tm, SlabGrad& g) {
-    auto over = [](float a, float b) { return kDualSteps ? a * (1.0f / b) : a / b; };
     const float w_raw = frequency_hz * (float)kTwoPi;
     const float omega = fmaxf(w_raw, kSmallEpsF);
-    const float wl_raw = over((float)kC0, frequency_hz);
+    const float wl_raw = (float)kC0 / frequency_hz;
     const float wavelength = fmaxf(wl_raw, kSmallEpsF);
     const float ca = fabsf(cos_theta);
     const float ct = fminf(fmaxf(ca, kSmallEpsF), 1.0f);
@@ -160,10 +124,10 @@ WC_HD void slab_fresnel_adj(float cos_theta, float eps_r, float sigma_e, float m
     const float eps = fmaxf(eps_r, kSmallEpsF);
     const float sig = fmaxf(sigma_e, 0.0f);
     const float mu = fmaxf(mu_r, kSmallEpsF);
-    const Cx<float> eta{eps, -over(sig, omega) * (float)(1.0 / kEps0)};
+    const Cx<float> eta{eps, -(sig / omega) * (float)(1.0 / kEps0)};
     const Cx<float> z{eta.re * mu - sin2, eta.im * mu};
-    const Cx<float> root = kDualSteps ? vq(csqrt(lq(z))) : csqrt(z);
-    const float q_scale = over(fmaxf(thickness, 0.0f) * (float)kTwoPi, wavelength);
+    const Cx<float> root = csqrt(z);
+    const float q_scale = fmaxf(thickness, 0.0f) * (float)kTwoPi / wavelength;
     const Cx<float> ph = scale(cexpj(-(root.re * q_scale * 2.0f)), expf(root.im * q_scale * 2.0f));
     const Cx<float> one{1.0f, 0.0f};
     const Cx<float> one_ph = one - ph;
@@ -210,7 +174,6 @@ WC_HD void slab_fresnel_adj(float cos_theta, float eps_r, float sigma_e, float m
 // reflected field and direction; adds to those of the incoming field (returned
 // in g_value), the incident direction, the normal and the slab parameters
 // (grad.ct is scratch).
-template <bool kDualSteps>
 WC_HD void reflect_c3_adj(const C3<float>& value, const V3<float>& incident, const V3<float>& normal_in, float eps_r,
                           float sigma_e, float mu_r, float gain, float thickness, float frequency_hz,
                           const C3<float>& g_out, const V3<float>& g_dir, C3<float>& g_value, V3<float>& g_inc,
@@ -226,15 +189,14 @@ WC_HD void reflect_c3_adj(const C3<float>& value, const V3<float>& incident, con
     const V3<float> p_in = safe_normalize(cross(s, incident), stable_perp_basis(incident, s));
     const V3<float> p_out = safe_normalize(cross(s, refl), stable_perp_basis(refl, s));
     Cx<float> te, tm;
-    if (kDualSteps) slab_value(fabsf(din), eps_r, sigma_e, mu_r, gain, thickness, frequency_hz, te, tm);
-    else slab_fresnel(fabsf(din), eps_r, sigma_e, mu_r, gain, thickness, frequency_hz, te, tm);
+    slab_fresnel(fabsf(din), eps_r, sigma_e, mu_r, gain, thickness, frequency_hz, te, tm);
     const Cx<float> e_s = c3_dot_real(value, s), e_p = c3_dot_real(value, p_in);
     // out = s (te e_s) + p_out (tm e_p)
     const Cx<float> g_ts = c3_dot_real(g_out, s), g_tp = c3_dot_real(g_out, p_out);
     V3<float> g_s = c3_axis_adj(g_out, te * e_s);
     const V3<float> g_po = c3_axis_adj(g_out, tm * e_p);
     grad.ct = 0.0f;
-    slab_fresnel_adj<kDualSteps>(fabsf(din), eps_r, sigma_e, mu_r, gain, thickness, frequency_hz, cmulj(e_s, g_ts),
+    slab_fresnel_adj(fabsf(din), eps_r, sigma_e, mu_r, gain, thickness, frequency_hz, cmulj(e_s, g_ts),
                      cmulj(e_p, g_tp), grad);
     const Cx<float> g_es = cmulj(te, g_ts), g_ep = cmulj(tm, g_tp);
     g_value = c3_axis(s, g_es) + c3_axis(p_in, g_ep);

@@ -483,7 +483,7 @@ __global__ void __launch_bounds__(128) refl_vjp_kernel(int n, ReflIn in, double 
             const bool turned = g_out.x != 0.0f || g_out.y != 0.0f || g_out.z != 0.0f;
             if (live || turned) {
                 C3<float> g_in;
-                reflect_c3_adj<false>(val_in[b], inc[b], nrm[b], in.eps[k], in.sig[k], in.mu[k], in.gain[k], in.thick[k], f,
+                reflect_c3_adj(val_in[b], inc[b], nrm[b], in.eps[k], in.sig[k], in.mu[k], in.gain[k], in.thick[k], f,
                                g_value, g_out, g_in, g_inc, g_nrm, sg);
                 g_value = g_in;
             }

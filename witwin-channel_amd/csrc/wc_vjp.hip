@@ -12,7 +12,6 @@
 // tiles (in tile order) gives dL/d(eps_r, sigma) per material, dL/df and
 // dL/d(tx position) per transmitter.
 #include "wc_api_internal.h"
-#include "wc_path_adjoint.h"
 #include "wc_tangent.h"
 #include "../../include/wcmi.h"
 
@@ -393,93 +392,63 @@ struct GeoGrad {
 template <int DM> struct LanePlanes {
     int depth;
     int group[DM];
-    PlaneGrad<DM> d;
+    float d[DM][4];  // dL / d(normal xyz, offset)
 };
 
+constexpr int kGeoTangents = 8;
+using DG = Dual<kGeoTangents>;
+
+__device__ __forceinline__ DG geo_seed(float v, int slot, int pass) {
+    const int local = slot - pass * kGeoTangents;
+    return seed<kGeoTangents>(v, (local >= 0 && local < kGeoTangents) ? local : -1);
+}
+
 // Geometry adjoint of one stored line-of-sight, reflection or transmission
-// path: one reverse sweep gives the gradients of all its planes (eight dual
-// tangents, 4 per plane, took depth / 2 evaluations in 3 KB of private memory).
-// Line-of-sight paths have no geometry (depth 0). Bound by the atomics: on the
-// heightfield (32,738 triangles, 125 k paths of depth 2) 696 us with dual
-// tangents and one atomic per lane, 547 us with the sweep, 148 us with the
-// groups' lanes summed first (flush_planes). Error against 64 bits as the dual
-// numbers': 2.9e-5 for coherent planes, 3.2e-5 for wall normals.
+// path: the recomputation with the planes carrying the tangents, 4 per
+// reflecting or transmitted plane, two planes a pass. Line-of-sight paths have
+// no geometry (depth 0). Bound by the tangents' private memory: on the
+// heightfield (32,738 triangles, 125 k paths of depth 2) 287 us, 696 us while
+// every lane added its own atomics (flush_planes). A reverse sweep of the same
+// paths in registers took 145 us and was no farther from 64 bits, path by path,
+// but rounds elsewhere: over 900 terrain maps its vertex gradients differed
+// from these by up to 4.8e-5 (three by more than 3e-5), where the two sums
+// (per lane, per group) of these differ by 2.2e-5 at most.
 template <int DM>
-__device__ __forceinline__ void geometry_path(const SceneView& s, const wc_solve& q, const wc_adjoint& ga, int t,
-                                              int cell, int desc, LanePlanes<DM>& out) {
-    const int comp = desc >> 24, cand = desc & 0xFFFFFF;
+__device__ void geometry_path(const SceneView& s, const wc_solve& q, const wc_adjoint& ga, int t, int cell, int desc,
+                              LanePlanes<DM>& out) {
     out.depth = 0;
-    if (comp != kCidRefl && comp != kCidTrans) return;
-    const CellAdjoint adj = cell_adjoint(ga, q, cell);
-    const int slot = slot_of_component(comp);
-    PathCotangent w;
-    w.coherent = adj.coherent;
-    w.a = {adj.a_re[slot], adj.a_im[slot]};
-    w.inc = 2.0f * adj.g_inc[slot] + adj.g_f_inc;
-    w.sp = sqrtf(fmaxf(q.tx_power[t], 0.0f));
-    const V3<float> tx = ld3(q.tx_pos + 3 * t), tx_pol = ld3(q.tx_pol + 3 * t);
-    const int rx_index = q.rx_shared ? cell - q.cell_offset[t] : cell;
-    const V3<float> rx = ld3(q.rx_pos + 3 * rx_index);
-    const V3<float> rx_pol = ld3(q.rx_pol + 3 * (q.rx_pol_stride ? rx_index : 0));
-    const float freq = (float)q.frequency_hz;
-    const double k_d = q.frequency_hz * kTwoPi / kC0;
-    if (comp == kCidRefl) {
-        const int* cg = q.chain_groups + (size_t)cand * kMaxDepth;
-        const double* img = q.chain_images + (size_t)cand * kMaxDepth * 3;
-        int depth = 0, mat[DM];
+    PathSetup ps;
+    setup_path<kPhaseMain>(s, q, ga, t, cell, desc, ps);
+    if (ps.comp == kCidLos || ps.depth == 0) return;
+    const bool refl = ps.comp == kCidRefl;
+    out.depth = min(ps.depth, DM);
+    const int slots = 4 * out.depth;
+    for (int pass = 0; pass * kGeoTangents < slots; ++pass) {
+        V3<DG> nrm[kMaxDepth];
+        DG off[kMaxDepth];
+        for (int k = 0; k < ps.depth; ++k) {
+            double o;
+            const V3<float> n = to_f(group_normal(s, refl ? ps.groups[k] : ps.walls[k].group, o));
+            nrm[k] = {geo_seed(n.x, 4 * k, pass), geo_seed(n.y, 4 * k + 1, pass), geo_seed(n.z, 4 * k + 2, pass)};
+            off[k] = geo_seed((float)o, 4 * k + 3, pass);
+        }
+        V3<DG> arrival;
+        const C3<DG> field =
+            refl ? reflection_tangent_planes(s, ps.depth, ps.faces, nrm, off, ps.tx, ps.rx, ps.tx_pol, ps.freq,
+                                             ps.k_d, ps.length_d, arrival)
+                 : transmission_tangent_walls(s, ps.depth, ps.walls, nrm, ps.tx, ps.rx, ps.tx_pol, ps.freq, ps.k_d,
+                                              ps.length_d, arrival);
+        float d[kGeoTangents];
+        contract(field, arrival, ps.rx_pol, ps.sqrt_power, ps.slot_id, ps.adj, false, d);
 #pragma unroll
         for (int b = 0; b < DM; ++b) {
-            out.group[b] = cg[b];
-            if (out.group[b] >= 0 && depth == b) depth = b + 1;
-        }
-        if (depth == 0) return;
-        // interaction faces of the frozen chain (image back-projection only)
-        V3<double> next = to_d(rx);
-        double length_d = 0.0;
+            const int local = 4 * b - pass * kGeoTangents;
+            if (local < 0 || local >= kGeoTangents || b >= out.depth) continue;
+            out.group[b] = refl ? ps.groups[b] : ps.walls[b].group;
 #pragma unroll
-        for (int b = DM - 1; b >= 0; --b) {
-            if (b >= depth) continue;
-            const int g = out.group[b];
-            double off;
-            const V3<double> n = group_normal(s, g, off);
-            const V3<double> im{img[3 * b], img[3 * b + 1], img[3 * b + 2]};
-            if (b == depth - 1) length_d = norm(next - im);
-            const double si = dot(n, im) - off, sn = dot(n, next) - off;
-            const V3<double> h = im + (next - im) * (si / (si - sn));
-            const int f = face_containing(s, g, to_f(h), to_f(n));
-            mat[b] = s.face_material[f >= 0 ? f : s.group_faces[s.group_face_offset[g]]];
-            next = h;
+            for (int i = 0; i < 4; ++i) out.d[b][i] = local == 0 ? d[i] : d[4 + i];
         }
-        out.depth = depth;
-        reflection_planes<DM>(s, depth, out.group, mat, tx, rx, tx_pol, rx_pol, freq, k_d, length_d, w, out.d);
-        return;
     }
-    const V3<float> seg = rx - tx;
-    const float len = norm(seg);
-    if (!(len > 2.0f * kSegmentBias)) return;
-    Hit walls[kMaxHits];
-    const float eps = kSegmentBias / len;
-    const RayPre r = ray_setup(tx.x, tx.y, tx.z, seg.x, seg.y, seg.z);
-    const int wall_count = gather_hits(s, r, eps, 1.0f - eps, q.max_depth, walls);
-    const int depth = min(min(wall_count, q.max_depth), DM);
-    const double dist = norm(to_d(rx) - to_d(tx));
-    const V3<double> dir = (to_d(rx) - to_d(tx)) * (1.0 / dist);
-    double carrier = dist;
-#pragma unroll
-    for (int b = 0; b < DM; ++b) {
-        if (b >= depth) continue;
-        double off;
-        const V3<double> nd = group_normal(s, walls[b].group, off);
-        const double ct = fmin(fmax(fabs(dot(dir, nd)), 1e-6), 1.0);
-        out.group[b] = walls[b].group;
-        const int m = s.face_material[walls[b].face];
-        double wall = 0.0;
-        for (int l = 0; l < s.mat_layer_count[m]; ++l)
-            wall += fmax((double)s.layer_thickness[s.mat_layer_offset[m] + l], 0.0);
-        carrier -= wall * ct;
-    }
-    out.depth = depth;
-    straight_normals<DM>(s, depth, walls, tx, rx, tx_pol, rx_pol, freq, k_d, carrier, w, out.d);
 }
 
 __device__ __forceinline__ float wave_sum(float v) {
@@ -505,7 +474,7 @@ __device__ __forceinline__ void flush_planes(const LanePlanes<DM>& planes, doubl
 #pragma unroll
     for (int b = 0; b < DM; ++b) {
         const bool on = b < planes.depth;
-        const float v[4] = {planes.d.nrm[b].x, planes.d.nrm[b].y, planes.d.nrm[b].z, planes.d.off[b]};
+        const float* v = planes.d[b];
         unsigned long long left = __ballot(on), single = left;
 #pragma unroll 1
         for (int round = 0; round < 4 && left; ++round) {
